@@ -152,23 +152,29 @@ typedef struct vj_join_opts {
 } vj_join_opts;
 
 /* Kernel shapes (vj_join_opts.tile / .table). All joins of one pipeline (a
- * batch) share them. The planner takes the standard tile (the large one in
- * the region layout), and the wide table
- * when the standard one would need more than 14 radix bits (build sides over
- * 2^24 rows of 8-byte keys); vj_tune times the alternatives. */
+ * batch) share them. The planner takes the wide table for build sides over
+ * 2^15 rows (2^16 of keys over 8 bytes) that one pass of 11 bits can partition
+ * for it, and where the standard one would need more than 14 radix bits; the
+ * large tile in one pass and in the region layout, the standard one in two
+ * passes of the exact layout. vj_tune times the alternatives. */
 #define VJ_TILE_STANDARD 1   /* 512 threads x 6 rows (keys <= 8 bytes), x 4 (<= 16), x 2 (wider) */
 #define VJ_TILE_SMALL 2      /* 512 threads x 2 rows: more blocks for small tables */
 #define VJ_TILE_LARGE 3      /* 512 threads x 8 rows (keys <= 8 bytes), x 6 (<= 16), x 4 (wider): longer runs
-                                per digit; the planner's tile in the region layout */
+                                per digit; the planner's tile in the region layout and its name for the one
+                                pass of up to 11 bits, whose blocks take 4096 rows, or up to three times as many
+                                at 11 bits */
 #define VJ_TABLE_STANDARD 1  /* 512 threads (8 waves), up to four blocks per CU, LDS table of 2048 rows
                                 (keys <= 8 bytes) or 1024 rows */
 #define VJ_TABLE_WIDE 2      /* 1024 threads (16 waves), one block per CU, LDS table of 8192 rows
-                                (keys <= 8 bytes), 4096 (<= 24 bytes) or 2048 */
+                                (keys <= 8 bytes; 8960 where 2^11 partitions average over 7168), 4096
+                                (<= 24 bytes) or 2048 */
 
 /* Partition layouts (vj_join_opts.layout). The planner takes the exact one;
  * vj_tune times both for two-pass plans.
- * EXACT: a histogram read of the keys gives every row its exact destination
- * (partitions back to back; no device atomics).
+ * EXACT: a histogram read of the keys gives every partition its exact place
+ * (partitions back to back). Up to 11 radix bits in all, asked for as one pass
+ * or two, take one pass over the rows (unless the standard or the small tile
+ * is asked for); more take two.
  * REGIONS: no histogram read. Each partition gets a region of fixed capacity
  * (its mean size plus a margin of 32 standard deviations of a uniform spread,
  * about 1.2-2x the mean) and the radix passes reserve their runs in it with

@@ -122,6 +122,13 @@ Err ensure_pinned(vj_ctx *c, size_t bytes) {
 // --- planning ----------------------------------------------------------------
 
 
+// Arena sizes of a plan, as allocate() requests them (ensure() rounds each up
+// to kAlign; under a budget it adds nothing else).
+struct ArenaSizes {
+    uint64_t tuples = 0, counts = 0, base = 0, ptask = 0, meta = 0;
+    uint64_t sum() const { return tuples + counts + base + ptask + meta; }
+};
+
 struct Plan {
     std::vector<JobDesc> jobs;
     std::vector<JoinDesc> joins;
@@ -130,6 +137,8 @@ struct Plan {
     std::vector<size_t> fin_off, mid_off;  // byte offsets in the tuples arena (SIZE_MAX: none)
     std::vector<uint64_t> fin_rows, mid_rows;  // rows of each buffer (the region layout leaves gaps)
     bool regions = false;                  // region layout (every job has two passes)
+    bool fan = false;                      // one-pass form (every job at most kFanBits bits)
+    uint32_t fan_bins = 1;                 // partitions of the largest job in the one-pass form
     size_t tuples_bytes = 0;
     uint64_t counts_words = 0, base_words = 0, ptask_words = 0;
     uint64_t taskmap_cap = 0;  // entries of the task map (after the task prefixes in the ptask arena)
@@ -143,8 +152,19 @@ struct Plan {
     LaunchShape shape{};
     HashCfg hash{};
     int kb = 0;
-    std::vector<std::pair<uint32_t, vj_built *>> keeps;  // (job, table to fill)
+    // Kept build sides: the job, the table it fills and that table's description,
+    // which is written to it only when the plan is allocated (planning may
+    // look at a second plan of other radix bits)
+    struct Keep {
+        uint32_t job;
+        vj_built *to;
+        vj_built what;
+    };
+    std::vector<Keep> keeps;
     uint64_t keep_bytes = 0;
+    // Bytes admission counts and the arenas take under a budget: those of the
+    // two-pass form where the one-pass form (which needs less) runs in its place
+    ArenaSizes floor{};
     // meta layout
     size_t off_jobs = 0, off_joins = 0, off_cs = 0, off_hb0 = 0, off_pt0 = 0, off_pc0 = 0, upload_bytes = 0;
     size_t off_jtasks = 0, off_task0 = 0, off_count = 0, off_ctl = 0, meta_bytes = 0;
@@ -166,14 +186,32 @@ int need_bits(uint64_t nr, int cap) {
     return nr > target ? ceil_log2((nr + target - 1) / target) : 0;
 }
 
+// Radix bits of the one-pass form for nr build rows: at most 3/4 of a build
+// chunk per partition on average (the quarter left is 11 standard deviations of
+// an even spread for 2048-row tables), 0 where all rows fit one chunk so. The
+// wide block, one per CU, also wants two partitions per CU to share out
+// (`share`: this join's part of the pipeline's rows); more cost shorter runs in the pass and a table each in the probe (2^21 x 2^24
+// 8-byte keys, total us: 2^9 partitions 234, 2^10 255, 2^11 283; 2^18 x 2^21:
+// 2^7 86, 2^9 76, 2^10 90). Past 3/4 of the wide table at kFanBits, up to 8300
+// rows of the 8960-row table.
+int fan_bits(uint64_t nr, int kb, int table, double share = 1.0) {
+    const uint64_t target = (uint64_t)probe_cap(kb, table) * 3 / 4;
+    int need = nr > target ? ceil_log2((nr + target - 1) / target) : 0;
+    if (table && nr > target) need = std::max(need, std::min(ceil_log2((uint64_t)(512 * share)), ceil_log2(nr / 256)));
+    return need > kFanBits && table == 1 && kb <= 8 && nr <= (uint64_t)8300 << kFanBits ? kFanBits : need;
+}
+
 // Radix passes and bits for one join (the reference fixes one radix width
 // per level, join_provider.cuh:296-300, and recurses until a partition fits,
 // :569-571; here the partition target is half an LDS build chunk of the
 // pipeline's table shape).
-Err plan_bits(uint64_t nr, int kb, int table, const vj_join_opts *o, int *P, int *b1, int *b2) {
-    const int need = need_bits(nr, probe_cap(kb, table));
+// `share`: the plan may run in the one-pass form, so bits are counted by
+// fan_bits where they fit it (0: it may not).
+Err plan_bits(uint64_t nr, int kb, int table, const vj_join_opts *o, double share, int *P, int *b1, int *b2) {
+    int need = need_bits(nr, probe_cap(kb, table));
     int passes = o->passes;
     if (passes < -1 || passes > 2) return Err::make(VJ_ERR_INVALID_ARGUMENT, "passes must be -1, 0, 1 or 2");
+    if (share > 0 && passes != 1 && fan_bits(nr, kb, table, share) <= kFanBits) need = fan_bits(nr, kb, table, share);
     if (passes == -1) passes = need == 0 ? 0 : (need <= kMaxPassBits ? 1 : 2);
     if (o->bits1 < 0 || o->bits2 < 0 || o->bits1 > kMaxPassBits || o->bits2 > kMaxPassBits)
         return Err::make(VJ_ERR_UNSUPPORTED, "radix bits per pass must be 1..8");
@@ -207,6 +245,19 @@ Err check_pair(const vj_table *r, const vj_table *s) {
 // Bytes of a resident table of n rows.
 size_t built_bytes(uint64_t n, int nc, int kw, uint32_t b1, uint32_t b2) {
     return align_up((size_t)kw * n) * nc + align_up((size_t)4 * n) + align_up((size_t)4 * ((1u << (b1 + b2)) + 1));
+}
+
+// A resident table of `t` partitioned on (P, b1, b2), without memory yet.
+vj_built built_as(const vj_table *t, const vj_hash_opts &hash, int P, int b1, int b2) {
+    vj_built k;
+    k.n = t->n_rows;
+    k.n_cols = t->n_cols;
+    k.key_width = t->key_width;
+    k.key_signed = t->key_signed != 0;
+    k.hash = hash;
+    k.b1 = (uint32_t)b1;
+    k.b2 = (uint32_t)(P >= 2 ? b2 : 0);
+    return k;
 }
 
 Err alloc_built(vj_built *b) {
@@ -303,7 +354,7 @@ void add_job(Plan &pl, const vj_table *t, int P, int b1, int b2, uint32_t shift0
     jd.b1 = P >= 1 ? b1 : 0;
     jd.b2 = P >= 2 ? b2 : 0;
     jd.shift0 = shift0;
-    const uint32_t T = pass_tile(pl.kb, pl.shape.tile);
+    const uint32_t T = pl.fan ? fan_tile(pl.kb, pl.shape.fan_big) : pass_tile(pl.kb, pl.shape.tile);
     const uint32_t n1 = 1u << jd.b1, nb = 1u << (jd.b1 + jd.b2);
     jd.base_off = (uint32_t)pl.base_words;
     jd.end_off = jd.base_off + 1;
@@ -315,7 +366,21 @@ void add_job(Plan &pl, const vj_table *t, int P, int b1, int b2, uint32_t shift0
     const uint32_t job_index = (uint32_t)pl.jobs.size();
     uint32_t chunks = 0;
     uint64_t mid_rows = jd.n, fin_rows = jd.n;
-    if (pl.regions && jd.b2) {
+    if (pl.fan) {
+        // one-pass form: counters [groups][nb] (one group where the tiles are
+        // too few to share lines), histogram blocks a whole number per group
+        if (jd.b1 && jd.n) {
+            pl.any_part = true;
+            jd.p1_tiles = (uint32_t)(((uint64_t)jd.n + T - 1) / T);
+            jd.groups = jd.p1_tiles > kXcds ? kXcds : 1;
+            const uint64_t share = (uint64_t)pl.hist_blocks_target * jd.n / std::max<uint64_t>(pl.hist_rows_total, 1);
+            const uint64_t most = (jd.p1_tiles + jd.groups - 1) / jd.groups;  // a group's tiles
+            jd.nrow = jd.groups * (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((share + jd.groups - 1) / jd.groups, most));
+            jd.m1_off = pl.counts_words;
+            pl.counts_words += (uint64_t)jd.groups * nb;
+            pl.fan_bins = std::max(pl.fan_bins, nb);
+        }
+    } else if (pl.regions && jd.b2) {
         // region layout: no histogram rows, no column scans; counters m1
         // [2^b1][nseg] and m2 [2^(b1+b2)] (zeroed by k_region_reset)
         RegionShape rs;
@@ -390,7 +455,7 @@ void add_job(Plan &pl, const vj_table *t, int P, int b1, int b2, uint32_t shift0
             fin = pl.tuples_bytes;
             pl.tuples_bytes += bytes(fin_rows);
         }
-        if (jd.b2) {
+        if (jd.b2 && !pl.fan) {
             mid = pl.tuples_bytes;
             pl.tuples_bytes += bytes(mid_rows);
         }
@@ -461,13 +526,26 @@ uint64_t largest_build(const std::vector<JoinSpec> &specs) {
     return nr;
 }
 
+// Build+probe block for a build side of nr rows where the caller leaves it
+// open. One-pass form: the wide block, whose larger tables need fewer partitions
+// (total us, best of each: 2^20 x 2^24 8-byte keys 233 against 256 with the
+// standard one, 2^18 x 2^21 76 / 102, 2^16 x 2^20 70 / 77, 2^18 x 2^21 of
+// 4 x u32 95 / 115); below 2^15 rows (2^16 of keys over 8 bytes) the standard
+// one, whose smaller blocks start sooner (2^14 x 2^17: 46 / 47, 2^16 x 2^19 of
+// 4 x u32 60 / 67).
+int choose_table(uint64_t nr, int kb, bool fan) {
+    if (fan) return nr <= (kb <= 8 ? 1u << 15 : 1u << 16) ? 0 : 1;
+    return need_bits(nr, build_cap(kb)) > kMaxHistBits ? 1 : 0;
+}
+
 // Kernel shapes of a pipeline (one for all of its joins): the caller's, else
 // the autotuned ones of the size class of the batch's largest build, else
 // the wide table when a standard one would need more than kMaxHistBits bits
 // of partitioning to bring the largest build down to half a chunk per
 // partition; a tile left open (-1) becomes the large tile in the region
 // layout and the standard one otherwise (build_join_plan).
-Err choose_shapes(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_opts *o, const vj_ctx *c) {
+// With `fan`, first the smallest table whose partitions fit the one-pass form.
+Err choose_shapes(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_opts *o, const vj_ctx *c, bool fan) {
     VJ_TRY(check_shapes(o));
     const uint64_t nr = largest_build(specs);
     int tile = o->tile - 1, table = o->table - 1;  // -1: choose
@@ -478,10 +556,33 @@ Err choose_shapes(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_op
             if (table < 0) table = (int)((it->second >> 28) & 0xF);
         }
     }
-    if (table < 0) table = need_bits(nr, build_cap(pl.kb)) > kMaxHistBits ? 1 : 0;
+    if (table < 0) table = choose_table(nr, pl.kb, fan);
     pl.shape.tile = tile;
     pl.shape.table = table;
     return Err::ok();
+}
+
+// Whether a pipeline's plan is made for the one-pass form: neither the region
+// layout nor a two-pass tile shape is asked for, and the caller's radix bits,
+// every resident table's and those its largest build side needs fit one pass.
+bool may_fan(int kb, const std::vector<JoinSpec> &specs, const vj_join_opts *o) {
+    if (o->layout == VJ_LAYOUT_REGIONS || (o->tile != 0 && o->tile != VJ_TILE_LARGE)) return false;
+    if (o->passes == 2 && o->bits1 + o->bits2 > kFanBits) return false;
+    for (const JoinSpec &js : specs)
+        if (js.res && js.res->b1 + js.res->b2 > (uint32_t)kFanBits) return false;
+    const uint64_t nr = largest_build(specs);
+    return fan_bits(nr, kb, o->table == VJ_TABLE_STANDARD ? 0 : 1) <= kFanBits;
+}
+
+// Whether a pipeline runs in the one-pass form: the exact layout, no tile shape
+// asked for that belongs to the two-pass kernels, and every job of at most
+// kFanBits radix bits in all. Then one histogram and one pass do the work of
+// a histogram and two passes.
+bool choose_fan(const Plan &pl, const std::vector<std::array<int, 3>> &bits) {
+    if (pl.regions || (pl.shape.tile >= 0 && pl.shape.tile != 2)) return false;
+    for (const auto &b : bits)
+        if ((b[0] >= 1 ? b[1] : 0) + (b[0] >= 2 ? b[2] : 0) > kFanBits) return false;
+    return true;
 }
 
 bool same_hash(const vj_hash_opts &a, const vj_hash_opts &b) {
@@ -514,8 +615,23 @@ bool choose_regions(const Plan &pl, const std::vector<JoinSpec> &specs, const st
     return true;
 }
 
+// Probe rows per task in the one-pass form. Where the pipeline has two
+// partitions per wide block of the chip (one per standard block), a task is a whole partition (5/4 of the mean,
+// so that most are not cut) and its table is built once; with fewer partitions
+// each is cut into enough tasks, but none of fewer rows than the table has
+// (its price). Standard blocks take at most one walk per task.
+uint32_t fan_task_rows(const Plan &pl, uint64_t s_rows, uint64_t nr, uint64_t ns, int bits) {
+    const uint64_t blocks = 256u * (pl.shape.table ? 1 : 4);
+    const uint64_t whole = (ns >> bits) + (ns >> (bits + 2)) + 256, fair = s_rows / (pl.shape.table ? 2 * blocks : blocks);
+    uint64_t rows = std::max<uint64_t>({(uint64_t)1024, nr >> bits, std::min(whole, fair)});
+    rows = (rows + 1023) / 1024 * 1024;
+    if (rows > whole * 2 / 3) rows = std::max(rows, whole);
+    return (uint32_t)std::min<uint64_t>(rows, pl.shape.table ? 1u << 20 : (uint64_t)kProbeChunk);
+}
+
 Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_opts *o, const vj_ctx *c = nullptr,
-                    bool allow_regions = true) {
+                    bool allow_regions = true, bool allow_fan = true) {
+
     const vj_table *t0 = specs[0].s;
     VJ_TRY(check_table(t0));
     VJ_TRY(make_hash_cfg(&o->hash, t0, &pl.hash));
@@ -523,11 +639,13 @@ Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_
     pl.shape.hp = hash_path(pl.hash);
     pl.shape.kw = t0->key_width;
     pl.shape.nc = t0->n_cols;
+    pl.shape.cus = c ? c->cus : 256;  // sizing without a context: an MI355X
     for (const JoinSpec &js : specs)
         if (!js.res) VJ_TRY(check_table(js.r));
-    VJ_TRY(choose_shapes(pl, specs, o, c));
+    const bool fan = allow_fan && may_fan(pl.kb, specs, o);
+    VJ_TRY(choose_shapes(pl, specs, o, c, fan));
     for (const JoinSpec &js : specs) pl.hist_rows_total += (js.res ? 0 : js.r->n_rows) + js.s->n_rows;
-    pl.hist_blocks_target = 2u * (uint32_t)(c ? c->cus : 256);  // sizing without a context: an MI355X
+    pl.hist_blocks_target = 2u * (uint32_t)pl.shape.cus;
     // radix plan of every join: (passes, bits1, bits2)
     std::vector<std::array<int, 3>> bits(specs.size());
     for (size_t i = 0; i < specs.size(); i++) {
@@ -546,7 +664,8 @@ Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_
             b2 = (int)b->b2;
         } else {
             VJ_TRY(check_pair(js.r, js.s));
-            VJ_TRY(plan_bits(js.r->n_rows, pl.kb, pl.shape.table, o, &P, &b1, &b2));
+            const double share = (double)(js.r->n_rows + js.s->n_rows) / (double)std::max<uint64_t>(pl.hist_rows_total, 1);
+            VJ_TRY(plan_bits(js.r->n_rows, pl.kb, pl.shape.table, o, fan ? std::max(share, 1e-9) : 0.0, &P, &b1, &b2));
             if (c && o->passes == -1 && !o->bits1 && !o->bits2 && !c->tuned.empty()) {  // autotuned plan
                 auto it = c->tuned.find(tune_key(js.r->n_rows, pl.kb, pl.shape.hp));
                 if (it != c->tuned.end()) {
@@ -563,7 +682,21 @@ Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_
         }
     }
     pl.regions = choose_regions(pl, specs, bits, o, c, allow_regions);
-    if (pl.shape.tile < 0) pl.shape.tile = pl.regions ? 2 : 0;
+    pl.fan = fan && choose_fan(pl, bits);
+    if (pl.shape.tile < 0) pl.shape.tile = pl.regions || pl.fan ? 2 : 0;
+    uint64_t s_rows = 0;
+    if (pl.fan) {
+        int most = 0;
+        uint64_t fill = 0;  // mean build rows per partition of the fullest join
+        for (size_t i = 0; i < specs.size(); i++) {
+            const int t = (bits[i][0] >= 1 ? bits[i][1] : 0) + (bits[i][0] >= 2 ? bits[i][2] : 0);
+            most = std::max(most, t);
+            fill = std::max<uint64_t>(fill, (specs[i].res ? specs[i].res->n : specs[i].r->n_rows) >> t);
+            s_rows += specs[i].s->n_rows;
+        }
+        pl.shape.fan_big = most >= kFanBits;
+        if (pl.shape.table == 1 && pl.kb <= 8 && most == kFanBits && fill > (uint64_t)wide_cap(pl.kb) * 7 / 8) pl.shape.table = 2;
+    }
     for (size_t i = 0; i < specs.size(); i++) {
         const JoinSpec &js = specs[i];
         const int P = bits[i][0], b1 = bits[i][1], b2 = bits[i][2];
@@ -575,16 +708,9 @@ Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_
             jd.job_r = (uint32_t)pl.jobs.size();
             add_job(pl, js.r, P, b1, b2, 0, js.keep != nullptr);
             if (js.keep) {
-                vj_built *k = js.keep;
-                k->n = js.r->n_rows;
-                k->n_cols = js.r->n_cols;
-                k->key_width = js.r->key_width;
-                k->key_signed = js.r->key_signed != 0;
-                k->hash = o->hash;
-                k->b1 = (uint32_t)b1;
-                k->b2 = (uint32_t)(P >= 2 ? b2 : 0);
-                pl.keeps.push_back({jd.job_r, k});
-                pl.keep_bytes += built_bytes(k->n, k->n_cols, k->key_width, k->b1, k->b2);
+                const vj_built k = built_as(js.r, o->hash, P, b1, b2);
+                pl.keeps.push_back({jd.job_r, js.keep, k});
+                pl.keep_bytes += built_bytes(k.n, k.n_cols, k.key_width, k.b1, k.b2);
             }
         }
         if (js.s->n_cols != t0->n_cols || js.s->key_width != t0->key_width ||
@@ -596,7 +722,8 @@ Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_
         jd.out_s = js.out_s;
         jd.cap = js.cap;
         jd.cap_r = probe_cap(pl.kb, pl.shape.table);
-        jd.cap_s = kProbeChunk;
+        jd.cap_s = pl.fan ? fan_task_rows(pl, s_rows, js.res ? js.res->n : js.r->n_rows, js.s->n_rows, (P >= 1 ? b1 : 0) + (P >= 2 ? b2 : 0))
+                          : kProbeChunk;
         jd.nparts = 1u << (P >= 1 ? b1 : 0) << (P >= 2 ? b2 : 0);
         jd.ptask_off = (uint32_t)pl.ptask_words;
         pl.ptask_words += jd.nparts + 1;
@@ -612,16 +739,11 @@ Err build_join_plan(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_
     return Err::ok();
 }
 
-// Arena sizes of a plan, as allocate() requests them (ensure() rounds each up
-// to kAlign; under a budget it adds nothing else).
-struct ArenaSizes {
-    uint64_t tuples, counts, base, ptask, meta;
-    uint64_t sum() const { return tuples + counts + base + ptask + meta; }
-};
 ArenaSizes arena_sizes(const Plan &pl) {
-    return {align_up(std::max<size_t>(pl.tuples_bytes, kAlign)), align_up(std::max<size_t>(pl.counts_words * 4, kAlign)),
-            align_up(std::max<size_t>(pl.base_words * 4, kAlign)),
-            align_up(std::max<size_t>((pl.ptask_words + pl.taskmap_cap) * 8, kAlign)), align_up(pl.meta_bytes)};
+    auto size = [](uint64_t bytes, uint64_t floor) { return align_up(std::max<size_t>({(size_t)bytes, (size_t)floor, kAlign})); };
+    return {size(pl.tuples_bytes, pl.floor.tuples), size(pl.counts_words * 4, pl.floor.counts),
+            size(pl.base_words * 4, pl.floor.base), size((pl.ptask_words + pl.taskmap_cap) * 8, pl.floor.ptask),
+            size(pl.meta_bytes, pl.floor.meta)};
 }
 
 uint64_t plan_scratch_bytes(const Plan &pl) { return arena_sizes(pl).sum(); }
@@ -642,6 +764,28 @@ Err admit(vj_ctx *c, const Plan &pl, uint64_t extra) {
                           std::max<uint64_t>(c->base.bytes, a.base) + std::max<uint64_t>(c->ptask.bytes, a.ptask) +
                           std::max<uint64_t>(c->meta.bytes, a.meta);
     if (keep + extra > c->budget) free_all(c);
+    return Err::ok();
+}
+
+// The plan of a pipeline. `bounded`: its memory is limited (a budget, the
+// fixed scratch), and what is admitted is the two-pass form's need, whichever
+// form runs: admission does not depend on the form a size happens to take. The
+// one-pass form needs no more in any arena; where it would, the two-pass form
+// runs.
+Err plan_joins(Plan &pl, const std::vector<JoinSpec> &specs, const vj_join_opts *o, const vj_ctx *c, bool allow_regions,
+               bool bounded) {
+    VJ_TRY(build_join_plan(pl, specs, o, c, allow_regions));
+    if (!bounded || !pl.fan) return Err::ok();
+    Plan two;
+    VJ_TRY(build_join_plan(two, specs, o, c, allow_regions, false));
+    const ArenaSizes f = arena_sizes(pl), t = arena_sizes(two);
+    if (f.tuples > t.tuples || f.counts > t.counts || f.base > t.base || f.ptask > t.ptask || f.meta > t.meta ||
+        pl.keep_bytes > two.keep_bytes) {
+        pl = std::move(two);
+        return Err::ok();
+    }
+    pl.floor = t;
+    pl.keep_bytes = two.keep_bytes;
     return Err::ok();
 }
 
@@ -680,21 +824,23 @@ uint64_t grown_with_slack(const vj_ctx *c, const ArenaSizes &a) {
 Err allocate(vj_ctx *c, Plan &pl, bool budget_slack = false, uint64_t extra = 0) {
     const bool slack =
         c->budget == 0 || (budget_slack && grown_with_slack(c, arena_sizes(pl)) + extra <= c->budget);
-    VJ_TRY(ensure(c->tuples, std::max<size_t>(pl.tuples_bytes, kAlign), slack));
-    VJ_TRY(ensure(c->counts, std::max<size_t>(pl.counts_words * 4, kAlign), slack));
-    VJ_TRY(ensure(c->base, std::max<size_t>(pl.base_words * 4, kAlign), slack));
-    VJ_TRY(ensure(c->ptask, std::max<size_t>((pl.ptask_words + pl.taskmap_cap) * 8, kAlign), slack));
-    VJ_TRY(ensure(c->meta, pl.meta_bytes, slack));
+    const ArenaSizes sz = arena_sizes(pl);
+    VJ_TRY(ensure(c->tuples, sz.tuples, slack));
+    VJ_TRY(ensure(c->counts, sz.counts, slack));
+    VJ_TRY(ensure(c->base, sz.base, slack));
+    VJ_TRY(ensure(c->ptask, sz.ptask, slack));
+    VJ_TRY(ensure(c->meta, sz.meta, slack));
     VJ_TRY(ensure_pinned(c, pl.meta_bytes));
     place_tuples(pl, static_cast<char *>(c->tuples.p));
     // kept build sides: their own allocation receives the last pass and the bases
     for (auto &kp : pl.keeps) {
-        vj_built *b = kp.second;
+        vj_built *b = kp.to;
         if (!b->mem) {
+            *b = kp.what;
             b->device = c->device;
             VJ_TRY(alloc_built(b));
         }
-        JobDesc &jd = pl.jobs[kp.first];
+        JobDesc &jd = pl.jobs[kp.job];
         for (int cc = 0; cc < 4; cc++) jd.fin_cols[cc] = b->cols[cc];
         jd.fin_ids = b->ids;
         jd.keep_base = b->base;
@@ -743,6 +889,11 @@ PipeArgs make_args(const Arenas &ar, const Plan &pl) {
     a.max_hist_bins = pl.max_hist_bins;
     a.pass_tile = pass_tile(pl.kb, pl.shape.tile);
     a.regions = pl.regions ? 1u : 0u;
+    if (pl.fan) {
+        a.pass_tile = fan_tile(pl.kb, pl.shape.fan_big);
+        a.fan_bins = pl.fan_bins;
+        a.count_words = pl.counts_words;
+    }
     a.hash = pl.hash;
     return a;
 }
@@ -786,6 +937,15 @@ Err launch_stages(vj_ctx *c, const Plan &pl, const PipeArgs &a, hipStream_t s, b
         VJ_LAUNCH(launch_pass(a, pl.shape, 2, s));
         if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_P2], s));
         VJ_LAUNCH(launch_tasks(a, s));
+    } else if (pl.fan) {
+        VJ_LAUNCH(launch_fan_reset(a, s));
+        VJ_LAUNCH(launch_fan_hist(a, pl.shape, s));
+        if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_HIST], s));
+        VJ_LAUNCH(launch_fan_plan(a, s));
+        if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_SCAN], s));
+        VJ_LAUNCH(launch_fan(a, pl.shape, s));
+        if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_P1], s));
+        if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_P2], s));
     } else {
         if (pl.any_part) VJ_LAUNCH(launch_hist(a, pl.shape, s));
         if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_HIST], s));
@@ -808,7 +968,8 @@ std::vector<uint64_t> graph_signature(const vj_ctx *c, const Plan &pl, const Pip
     std::vector<uint64_t> sig((sizeof(PipeArgs) + 7) / 8 + 10, 0);  // zeroed: PipeArgs padding is zero too
     memcpy(sig.data(), &a, sizeof(PipeArgs));
     uint64_t *x = sig.data() + (sizeof(PipeArgs) + 7) / 8;
-    x[0] = (uint64_t)pl.any_part | (uint64_t)pl.any_p2 << 1 | (uint64_t)pl.regions << 2;
+    x[0] = (uint64_t)pl.any_part | (uint64_t)pl.any_p2 << 1 | (uint64_t)pl.regions << 2 | (uint64_t)pl.fan << 3 |
+           (uint64_t)pl.shape.fan_big << 4;
     x[1] = (uint64_t)pl.shape.hp | (uint64_t)pl.shape.kw << 8 | (uint64_t)pl.shape.nc << 16 |
            (uint64_t)pl.shape.tile << 24 | (uint64_t)pl.shape.table << 32;
     x[2] = (uint64_t)c->cus * (uint64_t)probe_blocks_per_cu(pl.shape);
@@ -886,7 +1047,7 @@ void stage_bytes(const Plan &pl, uint64_t matches, vj_join_summary &s) {
             if (!pl.regions) s.bytes_histogram += n * kb;
             s.bytes_pass1 += n * (kb + ids_in) + n * (kb + 4);
         }
-        if (jd.b2 && !resident) s.bytes_pass2 += 2 * n * (kb + 4);
+        if (jd.b2 && !resident && !pl.fan) s.bytes_pass2 += 2 * n * (kb + 4);
         s.bytes_build_probe += jd.b1 || resident ? n * (kb + 4) : n * (kb + ids_in);
     }
     s.bytes_build_probe += matches * 8;
@@ -952,7 +1113,7 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
               std::vector<uint64_t> &counts, bool grow, uint64_t extra_bytes, int *retries_out,
               GraphMode gmode = GRAPH_OFF) {
     Plan pl;
-    VJ_TRY(build_join_plan(pl, specs, o, c));
+    VJ_TRY(plan_joins(pl, specs, o, c, true, c->budget != 0));
     VJ_TRY(admit(c, pl, extra_bytes + pl.keep_bytes));
     VJ_TRY(allocate(c, pl));
     PipeArgs a = make_args(ctx_arenas(c), pl);
@@ -1085,7 +1246,7 @@ namespace vj {
 
 Err pipeline_bytes(const std::vector<JoinSpec> &specs, const vj_join_opts *o, uint64_t *bytes) {
     Plan pl;
-    VJ_TRY(build_join_plan(pl, specs, o, nullptr, false));
+    VJ_TRY(build_join_plan(pl, specs, o, nullptr, false, false));
     // a lane launches under a budget: its arenas hold at least these sizes,
     // and growth slack only where the budget leaves room for it
     *bytes = plan_scratch_bytes(pl) + pl.keep_bytes;
@@ -1096,7 +1257,7 @@ Err pipeline_launch(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts 
                     size_t *count_off) {
     VJ_TRY(set_device(c));
     Plan pl;
-    VJ_TRY(build_join_plan(pl, specs, o, c, false));  // served batches complete asynchronously: exact layout
+    VJ_TRY(plan_joins(pl, specs, o, c, false, budget != 0));  // served batches complete asynchronously: exact layout
     c->budget = budget;
     VJ_TRY(admit(c, pl, pl.keep_bytes));
     VJ_TRY(allocate(c, pl, true, pl.keep_bytes));
@@ -1255,7 +1416,7 @@ vj_status vj_join_into_noalloc(vj_ctx *c, const vj_table *build, const vj_table 
     hipStream_t s = (hipStream_t)stream;
     std::vector<JoinSpec> specs{{build, probe, out_build, out_probe, capacity}};
     Plan pl;
-    e = build_join_plan(pl, specs, opts, c, false);  // exact layout: its scratch is bounded by the join's rows
+    e = plan_joins(pl, specs, opts, c, false, true);  // exact layout: its scratch is bounded by the join's rows
     if (e.failed()) return fail(c, e);
     // the arenas, laid out back to back in the fixed scratch
     const ArenaSizes az = arena_sizes(pl);
@@ -1505,11 +1666,21 @@ vj_status vj_build(vj_ctx *c, const vj_table *build, const vj_join_opts *opts, v
         pl.shape.hp = hash_path(pl.hash);
         pl.shape.kw = build->key_width;
         pl.shape.nc = build->n_cols;
+        pl.shape.cus = c->cus;
         e = check_shapes(opts);
         if (!e.failed()) {
+            std::vector<JoinSpec> specs{{build, nullptr, nullptr, nullptr, 0}};
+            const bool fan = !c->budget && may_fan(pl.kb, specs, opts);  // (a budget: see plan_joins)
             pl.shape.tile = opts->tile ? opts->tile - 1 : 0;
-            pl.shape.table = opts->table ? opts->table - 1 : (need_bits(build->n_rows, build_cap(pl.kb)) > kMaxHistBits ? 1 : 0);
-            e = plan_bits(build->n_rows, pl.kb, pl.shape.table, opts, &P, &b1, &b2);
+            pl.shape.table = opts->table ? opts->table - 1 : choose_table(build->n_rows, pl.kb, fan);
+            e = plan_bits(build->n_rows, pl.kb, pl.shape.table, opts, fan ? 1.0 : 0.0, &P, &b1, &b2);
+            const int bits = (P >= 1 ? b1 : 0) + (P >= 2 ? b2 : 0);
+            pl.fan = fan && bits <= kFanBits;
+            if (pl.fan) {
+                pl.shape.fan_big = bits >= kFanBits;
+                pl.hist_rows_total = build->n_rows;
+                pl.hist_blocks_target = 2u * (uint32_t)c->cus;
+            }
         }
     }
     if (!e.failed()) {
@@ -1519,16 +1690,9 @@ vj_status vj_build(vj_ctx *c, const vj_table *build, const vj_join_opts *opts, v
             b2 = 0;
         }
         add_job(pl, build, P, b1, b2, 0, true);
-        b->n = build->n_rows;
-        b->n_cols = build->n_cols;
-        b->key_width = build->key_width;
-        b->key_signed = build->key_signed != 0;
-        b->hash = opts->hash;
-        b->b1 = (uint32_t)b1;
-        b->b2 = (uint32_t)(P >= 2 ? b2 : 0);
-        b->device = c->device;
-        pl.keeps.push_back({0u, b});
-        pl.keep_bytes = built_bytes(b->n, b->n_cols, b->key_width, b->b1, b->b2);
+        const vj_built what = built_as(build, opts->hash, P, b1, b2);
+        pl.keeps.push_back({0u, b, what});
+        pl.keep_bytes = built_bytes(what.n, what.n_cols, what.key_width, what.b1, what.b2);
         finish_layout(pl);
         e = admit(c, pl, pl.keep_bytes);
     }
@@ -1632,6 +1796,14 @@ vj_status vj_tune(vj_ctx *c, const vj_table *build, const vj_table *probe, const
         const int cap = probe_cap(kb, table);
         const int need = need_bits(nr, cap);
         if (nr <= (uint64_t)cap) add({0, 0, 0, tile0, table, VJ_LAYOUT_EXACT});
+        const int fan = fan_bits(nr, kb, table);  // plans of the one-pass form (the large tile's name)
+        if (!opts->tile || opts->tile == VJ_TILE_LARGE) {
+            if (fan == 0) add({0, 0, 0, 2, table, VJ_LAYOUT_EXACT});
+            for (int tot = std::max(1, fan - 1); tot <= std::min(kFanBits, fan + 1); tot++) {
+                if (tot <= kMaxPassBits) add({1, tot, 0, 2, table, VJ_LAYOUT_EXACT});
+                else add({2, (tot + 1) / 2, tot / 2, 2, table, VJ_LAYOUT_EXACT});
+            }
+        }
         for (int b = std::max(1, need - 1); b <= std::min(kMaxPassBits, need + 1); b++)
             add({1, b, 0, tile0, table, VJ_LAYOUT_EXACT});
         for (int tot = std::max(2, need - 1); tot <= std::min(kMaxHistBits, need + 1); tot++)

@@ -227,10 +227,8 @@ __global__ __launch_bounds__(1024) void k_bases(PipeArgs a) {
 
 // One block of 1024 threads per join: build/probe tasks = R chunks x S chunks
 // of every partition pair, as an exclusive prefix over partitions.
-// The chunk capacities are powers of two (cap = 1 << log2), so the chunk
-// counts are shifts.
-__device__ __forceinline__ unsigned long long part_tasks(uint32_t nr, uint32_t ns, uint32_t lr, uint32_t ls) {
-    return nr && ns ? (unsigned long long)(((nr - 1) >> lr) + 1) * (((ns - 1) >> ls) + 1) : 0ull;
+__device__ __forceinline__ unsigned long long part_tasks(uint32_t nr, uint32_t ns, uint32_t cap_r, uint32_t cap_s) {
+    return nr && ns ? (unsigned long long)((nr - 1) / cap_r + 1) * ((ns - 1) / cap_s + 1) : 0ull;
 }
 
 // Task prefix, first kernel: one block per kTaskBlock partitions of a join.
@@ -296,8 +294,7 @@ __global__ __launch_bounds__(1024) void k_tasks(PipeArgs a) {
             to_global(a.base + js.end_off)[q] = q * js.region2 + ns;
         }
     }
-    const uint32_t lr = (uint32_t)__builtin_ctz(jd.cap_r), ls = (uint32_t)__builtin_ctz(jd.cap_s);
-    const unsigned long long t = ok ? part_tasks(nr, ns, lr, ls) : 0ull;
+    const unsigned long long t = ok ? part_tasks(nr, ns, jd.cap_r, jd.cap_s) : 0ull;
     unsigned long long total;
     const unsigned long long pre = block_excl_scan<unsigned long long, kTaskBlock / 64>(t, sh64, &total);
     if (ok) to_global(a.ptask + jd.ptask_off)[q] = pre;
@@ -354,6 +351,127 @@ __global__ __launch_bounds__(1024) void k_task_offsets(PipeArgs a) {
             a.task0[0] = 0;
             a.task0[1] = tasks;
             a.ctl->task_total = tasks;
+        }
+    }
+}
+
+// One-pass form, before the histogram: zeroes the count arena, the queue
+// ticket and the output counters.
+__global__ __launch_bounds__(1024) void k_fan_reset(PipeArgs a) {
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    if (i0 == 0) {
+        a.ctl->task_ticket = 0;
+        a.ctl->overflow = 0;
+    }
+    const gptr<uint32_t> c = to_global(a.counts);
+    for (uint64_t i = i0; i < a.count_words; i += step) c[i] = 0;
+    for (uint32_t j = i0; j < a.n_joins; j += step) a.out_count[j] = 0;
+}
+
+// One-pass form, between the histogram and the pass: one block per join turns
+// both sides' counts into partition bases and write cursors and writes the
+// join's task prefix (one join: also the queue totals and the task map). Two
+// partitions per thread; all loads of a side are in flight together, so the
+// kernel is two round trips and three block scans long (about 5 us), where
+// the two-pass form's column scans, bases and task prefix are four launches.
+__device__ void fan_side(const PipeArgs &a, const JobDesc &job, uint32_t *sh, uint32_t (&size)[2]) {
+    const uint32_t tid = threadIdx.x, nb = 1u << (job.b1 + job.b2), q0 = tid * 2;
+    const gptr<uint32_t> base = to_global(a.base + job.base_off), keep = to_global(job.keep_base);
+    size[0] = size[1] = 0;
+    if (job.b1 == 0) {  // not partitioned: one partition
+        if (tid == 0) {
+            base[0] = 0;
+            base[1] = size[0] = job.n;
+        }
+        return;
+    }
+    if (job.res_base) {  // resident: its bases are known
+        const gptr<const uint32_t> rb = to_global(job.res_base);
+        uint32_t x[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) x[k] = rb[q0 + k <= nb ? q0 + k : nb];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            if (q0 + k < nb) {
+                base[q0 + k] = x[k];
+                size[k] = x[k + 1] - x[k];
+            }
+        }
+        if (tid == 0) base[nb] = job.n;
+        return;
+    }
+    const gptr<uint32_t> cnt = to_global(a.counts + job.m1_off);
+    const uint32_t G = job.n ? job.groups : 0;  // an empty job has no counters
+    uint32_t c[2][kXcds];
+#pragma unroll
+    for (int g = 0; g < (int)kXcds; g++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const bool ok = (uint32_t)g < G && q0 + k < nb;
+            c[k][g] = ok ? cnt[(uint64_t)g * nb + q0 + k] : 0u;
+        }
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int g = 0; g < (int)kXcds; g++) size[k] += c[k][g];
+    uint32_t total;
+    uint32_t pre = block_excl_scan<uint32_t, kFanThreads / 64>(size[0] + size[1], sh, &total);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        if (q0 + k < nb) {
+            base[q0 + k] = pre;
+            if (keep) keep[q0 + k] = pre;
+            uint32_t cur = pre;
+#pragma unroll
+            for (int g = 0; g < (int)kXcds; g++) {
+                if ((uint32_t)g < G) cnt[(uint64_t)g * nb + q0 + k] = cur;
+                cur += c[k][g];
+            }
+        }
+        pre += size[k];
+    }
+    if (tid == 0) {
+        base[nb] = total;
+        if (keep) keep[nb] = total;
+    }
+}
+
+__global__ __launch_bounds__(kFanThreads) void k_fan_plan(PipeArgs a) {
+    __shared__ uint32_t sh32[kFanThreads / 64];
+    __shared__ unsigned long long sh64[kFanThreads / 64];
+    const uint32_t jn = blockIdx.x, tid = threadIdx.x, q0 = tid * 2;
+    uint32_t nr[2], ns[2];
+    if (a.n_joins == 0) {  // a build side alone (one job)
+        fan_side(a, a.jobs[jn], sh32, nr);
+        return;
+    }
+    const JoinDesc &jd = a.joins[jn];
+    const uint32_t n = jd.nparts;
+    fan_side(a, a.jobs[jd.job_r], sh32, nr);
+    fan_side(a, a.jobs[jd.job_s], sh32, ns);
+    const uint32_t cap_r = jd.cap_r, cap_s = jd.cap_s;
+    unsigned long long t[2], total;
+#pragma unroll
+    for (int k = 0; k < 2; k++) t[k] = part_tasks(nr[k], ns[k], cap_r, cap_s);
+    unsigned long long pre = block_excl_scan<unsigned long long, kFanThreads / 64>(t[0] + t[1], sh64, &total);
+    const gptr<unsigned long long> pt = to_global(a.ptask + jd.ptask_off), tmap = to_global(a.taskmap);
+    const bool one = a.n_joins == 1;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        if (q0 + k < n) {
+            pt[q0 + k] = pre;
+            if (one)
+                for (unsigned long long x = pre; x < pre + t[k] && x < a.taskmap_cap; x++) tmap[x] = q0 + k;
+        }
+        pre += t[k];
+    }
+    if (tid == 0) {
+        pt[n] = total;
+        a.join_tasks[jn] = total;
+        if (one) {
+            a.task0[0] = 0;
+            a.task0[1] = total;
+            a.ctl->task_total = total;
         }
     }
 }
@@ -449,6 +567,49 @@ hipError_t launch_region_reset(const PipeArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_fan_reset(const PipeArgs &a, hipStream_t s) {
+    const uint64_t blocks = (a.count_words + 4095) / 4096;
+    hipLaunchKernelGGL(k_fan_reset, dim3((unsigned)(blocks < 1 ? 1 : (blocks < 512 ? blocks : 512))), dim3(1024), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s) {
+    if (a.total_hist_blocks == 0) return hipSuccess;
+    switch (sh.hp) {
+    case HP_FNV: return StageLaunch<HP_FNV>::fan_hist(a, sh, s);
+    case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::fan_hist(a, sh, s);
+    case HP_GENERIC: return StageLaunch<HP_GENERIC>::fan_hist(a, sh, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s) {
+    if (a.total_p1_tiles == 0) return hipSuccess;
+    switch (sh.hp) {
+    case HP_FNV: return StageLaunch<HP_FNV>::fan(a, sh, s);
+    case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::fan(a, sh, s);
+    case HP_GENERIC: return StageLaunch<HP_GENERIC>::fan(a, sh, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+// The queue over several joins: prefix over their task totals, task map.
+static hipError_t launch_join_queue(const PipeArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(k_scan2, dim3(1), dim3(1024), 0, s, a);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && a.n_joins && a.taskmap_cap) {
+        hipLaunchKernelGGL(k_taskmap, dim3(a.n_joins, (a.max_nparts + 1023) / 1024), dim3(1024), 0, s, a);
+        e = hipGetLastError();
+    }
+    return e;
+}
+
+hipError_t launch_fan_plan(const PipeArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(k_fan_plan, dim3(a.n_joins ? a.n_joins : a.n_jobs), dim3(kFanThreads), 0, s, a);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess && a.n_joins > 1 ? launch_join_queue(a, s) : e;
+}
+
 hipError_t launch_tasks(const PipeArgs &a, hipStream_t s) {
     hipError_t e = hipSuccess;
     if (a.n_joins) {
@@ -459,13 +620,7 @@ hipError_t launch_tasks(const PipeArgs &a, hipStream_t s) {
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.n_joins == 1) return hipSuccess;  // k_tasks wrote the queue totals and the task map
-    hipLaunchKernelGGL(k_scan2, dim3(1), dim3(1024), 0, s, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (a.n_joins && a.taskmap_cap) {
-        hipLaunchKernelGGL(k_taskmap, dim3(a.n_joins, (a.max_nparts + 1023) / 1024), dim3(1024), 0, s, a);
-        e = hipGetLastError();
-    }
-    return e;
+    return launch_join_queue(a, s);
 }
 
 hipError_t launch_stage_copy(void *dst, const void *src, size_t bytes, hipStream_t s) {

@@ -5,6 +5,8 @@
 //            segment's pass-1 and (pass-1, pass-2) digit counts (LDS)
 //   k_pass   one radix pass over a tile (pass 1) or a (digit, segment) chunk
 //            (pass 2)
+//   k_fan_hist, k_fan  the one-pass form: counts per (group, partition), then
+//            one pass of up to 2^11 partitions with atomically reserved runs
 //   k_probe  persistent build + probe over (join, partition, R-chunk,
 //            S-chunk) tasks from a device queue
 //
@@ -377,6 +379,225 @@ __global__ __launch_bounds__(kPassThreads, (pass_waves_per_simd<HP, KW * NC, TV>
 }
 
 // ---------------------------------------------------------------------------
+// One-pass form
+// ---------------------------------------------------------------------------
+
+// Partition of a row: the pass-1 digit's bits above the pass-2 digit's, the
+// numbering two passes would give (b2 == 0: the one digit).
+__device__ __forceinline__ uint32_t fan_part(uint32_t h, uint32_t b1, uint32_t b2) {
+    return ((h & ((1u << b1) - 1)) << b2) | ((h >> b1) & ((1u << b2) - 1));
+}
+
+// Rows per (group, partition). Each block sweeps every nper-th tile of one
+// group with one LDS atomic per row, then adds its counters to the job's.
+// HBM-bound: the keys once.
+template <int HP, int KW, int NC>
+__global__ __launch_bounds__(kFanThreads, 8) void k_fan_hist(PipeArgs a) {
+    constexpr int KB = KW * NC;
+    constexpr int U = KB <= 16 ? 4 : 2;  // rows per thread in flight
+    extern __shared__ uint32_t lds[];    // [2^(b1+b2)]
+    const uint32_t tid = threadIdx.x, b = blockIdx.x;
+    const uint32_t j = upper_index(a.hist_block0, a.n_jobs, b);
+    const JobDesc &job = a.jobs[j];
+    const uint32_t b1 = job.b1, b2 = job.b2, nb = 1u << (b1 + b2), G = job.groups, n = job.n;
+    const uint32_t local = b - a.hist_block0[j], g = local & (G - 1), nper = job.nrow / G;
+    for (uint32_t q = tid; q < nb; q += kFanThreads) lds[q] = 0;
+    __syncthreads();
+    const GKeys<KW, NC> in = uniform_keys<KW, NC>(job.in);
+    const HashCfg hc = a.hash;
+    const uint32_t T = a.pass_tile, tiles = job.p1_tiles;
+    // the group's tiles: those whose index over the whole pipeline is g modulo the group count
+    for (uint32_t t = ((g - a.p1_tile0[j]) & (G - 1)) + G * (local / G); t < tiles; t += G * nper) {
+        const uint32_t lo = t * T, hi = lo + T < n ? lo + T : n;
+        for (uint32_t i0 = lo + tid; i0 < hi; i0 += kFanThreads * U) {
+            Key<KW, NC> key[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {  // all loads in flight at once (past the end: the first row again)
+                const uint32_t i = i0 + u * kFanThreads;
+                key[u] = load_key<KW, NC>(in, i < hi ? i : i0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (i0 + u * kFanThreads < hi) atomicAdd(&lds[fan_part(hash_key_lo<HP, KW, NC>(key[u], hc), b1, b2)], 1u);
+        }
+    }
+    __syncthreads();
+    uint32_t *cnt = a.counts + job.m1_off + (uint64_t)g * nb;
+    for (uint32_t q = tid; q < nb; q += kFanThreads) {
+        const uint32_t c = lds[q];
+        if (c) atomicAdd(cnt + q, c);
+    }
+}
+
+// Per tile: rank the rows by partition (one LDS counter per partition), reserve
+// each partition's run from the group's cursor, stage one column at a time in
+// LDS in partition order and write it out in runs. Persistent: as soon as a
+// column is staged its registers load the next tile's, so that the loads
+// cross the write-out (with one large block per CU nothing else would).
+// BIG: tile shape (fan_items).
+template <int HP, int KW, int NC, int BIG>
+__global__ __launch_bounds__(kFanThreads, (BIG || KW * NC > 16 ? 4 : 8)) void k_fan(PipeArgs a) {
+    using KT = typename KeyT<KW>::T;
+    constexpr int ITEMS = fan_items(KW * NC, BIG);
+    constexpr int T = kFanThreads * ITEMS, WAVES = kFanThreads / 64;
+    extern __shared__ __align__(16) unsigned char smem[];
+    KT *skeys = reinterpret_cast<KT *>(smem);            // [T] one column (then the row ids) at a time
+    uint32_t *sids = reinterpret_cast<uint32_t *>(smem);  // [T]
+    uint16_t *spart = reinterpret_cast<uint16_t *>(smem + (size_t)T * KW);        // [T]
+    uint32_t *cnt = reinterpret_cast<uint32_t *>(smem + (size_t)T * (KW + 2));    // [fan_bins] counts, then offsets
+    uint32_t *gdo = cnt + a.fan_bins;                                             // [fan_bins]
+    __shared__ uint32_t sh_scan[WAVES];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, total = a.total_p1_tiles;
+    const HashCfg hc = a.hash;
+    uint32_t b = blockIdx.x;  // tile over the whole pipeline; the grid is a multiple of kXcds: b stays on its XCD
+    if (b >= total) return;
+    uint32_t j = upper_index(a.p1_tile0, a.n_jobs, b);
+    uint32_t lo = (b - a.p1_tile0[j]) * T, n = a.jobs[j].n;
+    uint32_t rows = n - lo < (uint32_t)T ? n - lo : (uint32_t)T;
+    Key<KW, NC> key[ITEMS];
+    {
+        const GKeys<KW, NC> in = uniform_keys<KW, NC>(a.jobs[j].in);
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {  // every load in flight at once (past the end: row lo again)
+            const uint32_t i = it * kFanThreads + tid;
+            key[it] = load_key<KW, NC>(in, lo + (i < rows ? i : 0u));
+        }
+    }
+    for (uint32_t q = tid; q < a.fan_bins; q += kFanThreads) cnt[q] = 0;
+    __syncthreads();
+    while (true) {
+        const JobDesc &job = a.jobs[j];
+        const uint32_t b1 = job.b1, b2 = job.b2, nb = 1u << (b1 + b2);
+        // the next tile, whose columns are loaded on the way
+        const uint32_t b_next = b + gridDim.x;
+        const bool more = b_next < total;
+        uint32_t j_next = j;
+        if (more && b_next >= a.p1_tile0[j + 1]) j_next = upper_index(a.p1_tile0, a.n_jobs, b_next);
+        const uint32_t lo_next = more ? (b_next - a.p1_tile0[j_next]) * T : 0u, n_next = a.jobs[j_next].n;
+        const uint32_t rows_next = !more ? 0u : (n_next - lo_next < (uint32_t)T ? n_next - lo_next : (uint32_t)T);
+        const GKeys<KW, NC> in_next = uniform_keys<KW, NC>(a.jobs[j_next].in);
+        // 1. partition and rank of every row
+        uint32_t slot[ITEMS];  // partition | rank << kFanBits, then the row's slot in partition order
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {
+            const uint32_t q = fan_part(hash_key_lo<HP, KW, NC>(key[it], hc), b1, b2);
+            slot[it] = q;
+            if (it * kFanThreads + tid < rows) slot[it] |= atomicAdd(&cnt[q], 1u) << kFanBits;
+        }
+        __syncthreads();
+        // 2. each thread: its (two) partitions' runs reserved, their offsets in the tile
+        const uint32_t per = nb > (uint32_t)kFanThreads ? 2u : 1u, q0 = tid * per;
+        uint32_t c[2], got[2];
+        uint32_t *cur = a.counts + job.m1_off + (uint64_t)(b & (job.groups - 1)) * nb;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            c[k] = (uint32_t)k < per && q0 + k < nb ? cnt[q0 + k] : 0u;
+            got[k] = c[k] ? atomicAdd(cur + q0 + k, c[k]) : 0u;
+        }
+        uint32_t pre = wave_incl_scan(c[0] + c[1]);
+        if (lane == 63) sh_scan[w] = pre;
+        __syncthreads();
+        pre -= c[0] + c[1];
+#pragma unroll
+        for (int k = 0; k < WAVES; k++) pre += (uint32_t)k < w ? sh_scan[k] : 0u;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            if ((uint32_t)k < per && q0 + k < nb) {
+                cnt[q0 + k] = pre;
+                gdo[q0 + k] = got[k] - pre;  // output row of slot s = gdo[partition] + s
+                pre += c[k];
+            }
+        }
+        __syncthreads();
+        // 3. slots; the first key column staged with its rows' partitions
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {
+            if (it * kFanThreads + tid < rows) {
+                const uint32_t q = slot[it] & ((1u << kFanBits) - 1);
+                slot[it] = cnt[q] + (slot[it] >> kFanBits);
+                skeys[slot[it]] = key[it].c[0];
+                spart[slot[it]] = (uint16_t)q;
+            }
+        }
+        if (more) {  // block-uniform
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const uint32_t i = it * kFanThreads + tid;
+                key[it].c[0] = in_next.c[0][lo_next + (i < rows_next ? i : 0u)];
+            }
+        }
+        __syncthreads();
+        // 4. columns out in slot order; each thread keeps its slots' output rows
+        for (uint32_t q = tid; q < a.fan_bins; q += kFanThreads) cnt[q] = 0;
+        uint32_t dst[ITEMS];
+        {
+            const gptr<KT> out = uniform_global(static_cast<KT *>(job.fin_cols[0]));
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const uint32_t s = it * kFanThreads + tid;
+                if (s < rows) {
+                    dst[it] = gdo[spart[s]] + s;
+                    out[dst[it]] = skeys[s];
+                }
+            }
+        }
+#pragma unroll
+        for (int col = 1; col < NC; col++) {
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++)
+                if (it * kFanThreads + tid < rows) skeys[slot[it]] = key[it].c[col];
+            if (more) {
+#pragma unroll
+                for (int it = 0; it < ITEMS; it++) {
+                    const uint32_t i = it * kFanThreads + tid;
+                    key[it].c[col] = in_next.c[col][lo_next + (i < rows_next ? i : 0u)];
+                }
+            }
+            __syncthreads();
+            const gptr<KT> out = uniform_global(static_cast<KT *>(job.fin_cols[col]));
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const uint32_t s = it * kFanThreads + tid;
+                if (s < rows) out[dst[it]] = skeys[s];
+            }
+        }
+        // 5. the row ids
+        const gptr<const uint32_t> ids = uniform_global(job.in.rowids);
+        __syncthreads();
+        if (ids) {  // block-uniform
+            uint32_t id[ITEMS];
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const uint32_t i = it * kFanThreads + tid;
+                id[it] = ids[lo + (i < rows ? i : 0u)];
+            }
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++)
+                if (it * kFanThreads + tid < rows) sids[slot[it]] = id[it];
+        } else {
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++)
+                if (it * kFanThreads + tid < rows) sids[slot[it]] = lo + it * kFanThreads + tid;
+        }
+        __syncthreads();
+        const gptr<uint32_t> out = uniform_global(job.fin_ids);
+#pragma unroll
+        for (int it = 0; it < ITEMS; it++) {
+            const uint32_t s = it * kFanThreads + tid;
+            if (s < rows) out[dst[it]] = sids[s];
+        }
+        if (!more) return;
+        b = b_next;
+        j = j_next;
+        lo = lo_next;
+        rows = rows_next;
+        // the staging buffer is written again after three barriers of the next
+        // tile; its counters were cleared before the last two of this one
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Build + probe
 // ---------------------------------------------------------------------------
 
@@ -385,12 +606,12 @@ struct ProbeTask {
     uint32_t *out_r, *out_s;
     unsigned long long *count;
     uint64_t cap;
-    unsigned long long out_base;  // first output row of this task
+    unsigned long long out_base[4];  // first output row of walk k's matches (k & 3)
     uint32_t r_lo, r_n, s_lo, s_n;
-    uint32_t nslots, shift, one_based;
+    uint32_t nheads, hshift, shift, one_based;  // heads; 32 - their log2
     uint32_t dup;
     uint32_t done;
-    uint32_t wave_count[kMaxProbeWaves];
+    uint32_t wave_count[4][kMaxProbeWaves];  // matches per wave of walk k (k & 3)
     // the join whose fixed fields the record holds (~0: none yet), its
     // sides' partition start / end offsets in base, chunk sizes, first task
     // and per-partition task prefix
@@ -399,43 +620,29 @@ struct ProbeTask {
     const unsigned long long *pt;
 };
 
-constexpr int kProbeUnroll = 2;
-constexpr int kBucketSlots = 4;  // LDS table: buckets of 4 slots (one 16-byte load)
 
 // One task's parameters for the walks (all wave-uniform).
 struct WalkArgs {
     GView s;
-    gptr<const uint32_t> r_ids;  // build rows' ids (null: the row index)
-    uint32_t r_lo;
     gptr<uint32_t> out_r, out_s;
     uint64_t cap;
-    uint32_t s_lo, s_end, bmask, shift, ob1;
+    uint32_t s_lo, s_end, hshift, shift, ob1;
     bool dup;
 };
 
 __device__ __forceinline__ WalkArgs walk_args(const ProbeTask &t) {
     WalkArgs w;
     w.s = uniform_view(t.s);
-    w.r_ids = uniform_global(t.r.rowids);
-    w.r_lo = uniform(t.r_lo);
     w.out_r = uniform_global(t.out_r);
     w.out_s = uniform_global(t.out_s);
     w.cap = uniform((uint64_t)t.cap);
     w.s_lo = uniform(t.s_lo);
-    w.s_end = uniform(t.s_lo + t.s_n);
-    w.bmask = uniform((t.nslots >> 2) - 1);
+    w.s_end = w.s_lo + uniform(t.s_n < (uint32_t)kProbeChunk ? t.s_n : (uint32_t)kProbeChunk);
+    w.hshift = uniform(t.hshift);
     w.shift = uniform(t.shift);
     w.ob1 = uniform(t.one_based);
-    w.dup = uniform(t.dup) != 0;
+    w.dup = false;  // known once the table is built
     return w;
-}
-
-// Row id of build row o of the task's chunk, read from the partitioned build
-// side (its rows were just loaded by the build step, so the read is cached).
-// (IDS: from the table's copy in LDS, `rid`.)
-template <bool IDS> __device__ __forceinline__ uint32_t build_id(const WalkArgs &wa, const uint32_t *rid, uint32_t o) {
-    if constexpr (IDS) return rid[o];
-    return wa.r_ids ? wa.r_ids[wa.r_lo + o] : wa.r_lo + o;
 }
 
 // Writes a wave's matches straight to the join output: the matching lanes of
@@ -456,30 +663,48 @@ struct Emitter {
     }
 };
 
-// Walks over this wave's rows of the S chunk. The chunk holds up to
-// kProbeChunk = ITERS x TH x kProbeUnroll rows (TH threads per block, see
-// ProbeShape); in iteration `it` lane `l` of wave `w` owns rows
-// it*TH*U + w*64*U + u*64 + l.
-// The table holds one entry per distinct key (equal keys of the build chunk
-// are chained behind it, see the build step), so a row matches at most one
-// entry. probe_walk finds it, keeps its index in registers and counts the
-// row's matches (the chain length); replay_walk then writes them without
-// probing again. Probing runs in rounds: each round reads one whole bucket
-// for every unfinished row of the lane (U independent LDS chains per lane);
-// a round is branch-free (selects, no per-row branches). The S keys of the
-// next iteration are loaded before the current one is probed, so one HBM round
-// trip overlaps each iteration's probing (where registers allow, see PF).
+// The block's LDS table of one build chunk: chained hashing. heads[h] is the
+// first entry of chain h (0: none), key / id / nxt are indexed by entry
+// (entry = chunk row + 1). Entries 1.. only: entry 0 reads as an end.
+template <typename KT, int NC, int CAP> struct LdsTable {
+    KT *key;         // [NC][CAP + 1]
+    uint32_t *id;    // [CAP + 1]
+    uint16_t *nxt;   // [CAP + 1]
+    uint16_t *head;  // [heads]
+    __device__ __forceinline__ bool eq(uint32_t e, const KT (&k)[NC]) const {
+        bool r = true;
+#pragma unroll
+        for (int c = 0; c < NC; c++) r &= key[c * (CAP + 1) + e] == k[c];
+        return r;
+    }
+    __device__ __forceinline__ bool eq(uint32_t e, uint32_t f) const {
+        bool r = true;
+#pragma unroll
+        for (int c = 0; c < NC; c++) r &= key[c * (CAP + 1) + e] == key[c * (CAP + 1) + f];
+        return r;
+    }
+};
 
-// A key's place in the LDS table: its 16-bit tag (never 0) << 16 | its bucket,
-// from the low 32 hash bits above the partition digits (the digits are the
-// same for every row of a partition; digits and buckets end below bit 27).
-// The tag is the top of a multiplicative hash of those bits, which depends on
-// all of them (the top 16 bits of a 64-bit hash would not do: custom_xor_hw's
-// 64-bit hash of 4-byte keys has a zero upper half, so every key would get
-// the same tag).
-__device__ __forceinline__ uint32_t table_place(uint32_t lo, uint32_t shift, uint32_t bmask) {
-    const uint32_t y = lo >> shift;
-    return ((((y * 0x9E3779B1u) >> 16) | 1u) << 16) | (y & bmask);
+// Walks over this wave's rows of the S chunk. The chunk holds up to
+// kProbeChunk = ITERS x TH x U rows (TH threads per block, see ProbeShape); in
+// iteration `it` lane `l` of wave `w` owns rows it*TH*U + w*64*U + u*64 + l.
+// probe_walk finds each row's first matching entry, keeps it in registers and
+// counts the row's matches (equal keys further down the chain); replay_walk
+// then writes them. All U rows of a lane step down their chains together: one
+// key and one link per row and step, with selects instead of branches, until
+// the wave's longest chain ends (about three steps at four heads per row). A
+// step is some 8 VALU instructions per row; buckets of tags read whole took
+// about 35 per round and could not afford fewer than two slots per row.
+// The S keys of the next iteration are loaded before the current one is
+// probed, so one HBM round trip overlaps each iteration's probing (where
+// registers allow, see PF); nk holds the first iteration's, loaded by the caller.
+
+// A key's chain, from the low 32 hash bits above the partition digits (the
+// digits are the same for every row of a partition): the top bits of their
+// product with the golden ratio, which depend on all of them (FNV's low bits
+// depend only on the keys' low bits, and custom_xor_hw mixes less).
+__device__ __forceinline__ uint32_t chain_of(uint32_t lo, uint32_t shift, uint32_t hshift) {
+    return ((lo >> shift) * 0x9E3779B1u) >> hshift;
 }
 
 template <int N> __device__ __forceinline__ uint32_t res_get(const uint32_t (&r)[N], int k) {
@@ -493,10 +718,11 @@ template <int N> __device__ __forceinline__ void res_set(uint32_t (&r)[N], int k
 template <int PV> struct ProbeShape {
     static constexpr int TH = probe_threads(PV);
     static constexpr int WAVES = TH / 64;
-    static constexpr int ITERS = kProbeChunk / (TH * kProbeUnroll);
-    static constexpr int RES = ITERS * kProbeUnroll / 2;  // words of packed 16-bit results per lane
-    static_assert(kProbeUnroll % 2 == 0, "an iteration's results fill whole words");
-    static_assert(ITERS * TH * kProbeUnroll == kProbeChunk && WAVES <= kMaxProbeWaves, "probe chunk shape");
+    static constexpr int U = PV ? 4 : 2;  // rows per lane and iteration (the wide block has half the waves, twice the registers)
+    static constexpr int ITERS = kProbeChunk / (TH * U);
+    static constexpr int RES = ITERS * U / 2;  // words of packed 16-bit results per lane
+    static_assert(U % 2 == 0, "an iteration's results fill whole words");
+    static_assert(ITERS * TH * U == kProbeChunk && WAVES <= kMaxProbeWaves, "probe chunk shape");
 };
 
 // First S row of this lane in iteration `it` of a walk with U rows per lane.
@@ -523,149 +749,93 @@ template <int N> __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
     return v;
 }
 
-template <int HP, int KW, int NC, int PV>
-__device__ __forceinline__ uint32_t probe_walk(const WalkArgs &wa, const HashCfg &hc,
-                                               const typename KeyT<KW>::T *rk, const uint32_t *slots,
-                                               const uint16_t *nxt, uint32_t (&res)[ProbeShape<PV>::RES]) {
-    constexpr int CAP = probe_cap(KW * NC, PV);
+template <int HP, int KW, int NC, int PV, typename Tab>
+__device__ __forceinline__ uint32_t probe_walk(const WalkArgs &wa, const HashCfg &hc, const Tab &tab,
+                                               Key<KW, NC> (&nk)[ProbeShape<PV>::U],
+                                               uint32_t (&res)[ProbeShape<PV>::RES]) {
     constexpr int TH = ProbeShape<PV>::TH, ITERS = ProbeShape<PV>::ITERS;
-    constexpr int U = kProbeUnroll;
+    constexpr int U = ProbeShape<PV>::U;
     // Next-iteration loads double the key registers; they are used where the
     // kernel stays within its register budget (single 8-byte key, or the wide
     // block's 128 VGPRs; FNV / XOR).
-    constexpr bool PF = (KW * NC <= 8 || PV == 1) && HP != HP_GENERIC;
-    const uint32_t bmask = wa.bmask, shift = wa.shift, s_end = wa.s_end;
+    constexpr bool PF = (KW * NC <= 8 || PV != 0) && HP != HP_GENERIC;
+    const uint32_t hshift = wa.hshift, shift = wa.shift, s_end = wa.s_end;
     uint32_t total = 0;  // this lane's matches
-    Key<KW, NC> nk[U];
-    walk_load<U, TH, KW, NC>(wa, 0, nk);
 #pragma unroll
     for (int it = 0; it < ITERS; it++) {
         if (walk_wave_row<U, TH>(wa, it) >= s_end) break;  // wave-uniform
         const uint32_t row = walk_row<U, TH>(wa, it);
         Key<KW, NC> sk[U];
-        // 16-bit tag << 16 | first bucket (buckets < 2^16); round r reads bucket
-        // first + r. 0 once the row is done (or past the chunk): tag 0 matches
-        // only empty slots, so such a row finds nothing and stays done.
-        uint32_t st[U];
         if (!PF && it > 0) walk_load<U, TH, KW, NC>(wa, it, nk);
 #pragma unroll
         for (int u = 0; u < U; u++) sk[u] = nk[u];
         if (PF && it + 1 < ITERS) walk_load<U, TH, KW, NC>(wa, it + 1, nk);
+        uint32_t e[U], f[U];  // the row's next chain entry (0: done, or past the chunk); its match (0: none)
 #pragma unroll
-        for (int u = 0; u < U; u++)
-            st[u] = row + u * 64 < s_end ? table_place(hash_key_lo<HP, KW, NC>(sk[u], hc), shift, bmask) : 0u;
-        uint32_t rnd = 0;
+        for (int u = 0; u < U; u++) {
+            const uint32_t h = tab.head[chain_of(hash_key_lo<HP, KW, NC>(sk[u], hc), shift, hshift)];
+            e[u] = row + u * 64 < s_end ? h : 0u;
+            f[u] = 0;
+        }
         while (true) {
             uint32_t any = 0;
 #pragma unroll
-            for (int u = 0; u < U; u++) any |= st[u];
+            for (int u = 0; u < U; u++) any |= e[u];
             if (!__ballot(any != 0)) break;
-            uint4 E[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) E[u] = *reinterpret_cast<const uint4 *>(slots + (((st[u] + rnd) & bmask) << 2));
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const uint32_t tg = st[u] >> 16;
-                const uint32_t e4[kBucketSlots] = {E[u].x, E[u].y, E[u].z, E[u].w};
-                // the first entry whose tag matches (0: none; tags are never 0, so
-                // neither an entry nor a match is 0); a bucket's slots fill in
-                // order, so it has a free slot (the row's key cannot be further
-                // on) iff its last slot is free
-                uint32_t ej = 0;
-#pragma unroll
-                for (int j = kBucketSlots - 1; j >= 0; j--) ej = (e4[j] >> 16) == tg ? e4[j] : ej;
-                const bool emp = e4[kBucketSlots - 1] == 0;
-                uint32_t fo = ej ? (ej & 0xFFFFu) - 1 : 0u;
-                bool found = ej != 0;
-#pragma unroll
-                for (int c = 0; c < NC; c++) found &= rk[c * CAP + fo] == sk[u].c[c];
-                if (__ballot(ej != 0 && !found)) {  // a 16-bit tag collision: the later candidates, in slot order
-                    uint32_t cand = 0;
-#pragma unroll
-                    for (int j = 0; j < kBucketSlots; j++) cand |= ((e4[j] >> 16) == tg ? 1u : 0u) << j;
-                    cand = ej != 0 && !found ? cand & (cand - 1) : 0u;
-                    while (__ballot(cand != 0)) {
-                        const bool has = cand != 0;
-                        const uint32_t j = __builtin_ctz(cand | (1u << kBucketSlots));
-                        const uint32_t ejj = j == 0 ? e4[0] : (j == 1 ? e4[1] : (j == 2 ? e4[2] : e4[3]));
-                        cand &= cand - 1;
-                        const uint32_t o = has ? (ejj & 0xFFFFu) - 1 : 0u;
-                        bool eq = has;
-#pragma unroll
-                        for (int c = 0; c < NC; c++) eq &= rk[c * CAP + o] == sk[u].c[c];
-                        if (eq) {
-                            found = true;
-                            fo = o;
-                            cand = 0;
-                        }
-                    }
-                }
-                res[(it * U + u) >> 1] |= (found ? fo + 1 : 0u) << (((it * U + u) & 1) * 16);
-                uint32_t n = found ? 1u : 0u;
-                if (wa.dup) {  // wave-uniform: equal keys of the build chunk are chained behind the entry
-                    uint32_t x = found ? nxt[fo] : 0u;
-                    while (__ballot(x != 0)) {
-                        n += x != 0;
-                        x = x != 0 ? nxt[x - 1] : 0u;
-                    }
-                }
-                total += n;
-                st[u] = found || emp ? 0u : st[u];
+                const uint32_t nx = tab.nxt[e[u]];
+                const bool hit = tab.eq(e[u], sk[u].c) && e[u] != 0;
+                f[u] = hit && f[u] == 0 ? e[u] : f[u];
+                total += hit;
+                e[u] = hit && !wa.dup ? 0u : nx;  // equal keys in the chunk: to the chain's end
             }
-            rnd++;
         }
+#pragma unroll
+        for (int u = 0; u < U; u++) res[(it * U + u) >> 1] |= f[u] << (((it * U + u) & 1) * 16);
     }
     return wave_sum<64>(total);
 }
 
-// Writes the matches probe_walk kept: each matched row's entry, then (when the
-// build chunk has equal keys) the rest of its chain. The probe-side and
-// build-side row ids of a group of G iterations are loaded before any is
-// written, so their round trips overlap.
-template <int G, int PV, bool IDS>
-__device__ __forceinline__ void replay_walk(const WalkArgs &wa, const uint16_t *nxt, const uint32_t *rid,
-                                            const uint32_t (&res)[ProbeShape<PV>::RES], Emitter &em) {
-    constexpr int U = kProbeUnroll;
-    constexpr int TH = ProbeShape<PV>::TH, ITERS = ProbeShape<PV>::ITERS;
-    static_assert(ITERS % G == 0, "replay groups");
-    const uint32_t ob1 = wa.ob1, s_end = wa.s_end;
+// Row ids of this lane's rows of iterations g .. g + G, matched or not, with
+// clamped indexes: no per-row branches, and the loads are issued together (rows
+// past the chunk, and all rows of iterations the walk skipped, hold no match:
+// they read row s_lo).
+template <int G, int PV>
+__device__ __forceinline__ void load_ids(const WalkArgs &wa, int g, uint32_t (&sid)[G * ProbeShape<PV>::U]) {
+    constexpr int U = ProbeShape<PV>::U, TH = ProbeShape<PV>::TH;
 #pragma unroll
-    for (int g = 0; g < ITERS; g += G) {
-        if (walk_wave_row<U, TH>(wa, g) >= s_end) break;  // wave-uniform
-        // ids of every row, matched or not, with clamped indexes: no per-row
-        // branches, and the loads of a group are issued together (rows past
-        // the chunk, and all rows of iterations the walk skipped, hold no
-        // match: they read row s_lo / build row 0)
-        uint32_t sid[G * U], bid[G * U];
+    for (int it = 0; it < G; it++) {
+        const uint32_t row = walk_row<U, TH>(wa, g + it);
 #pragma unroll
-        for (int it = 0; it < G; it++) {
-            const uint32_t row = walk_row<U, TH>(wa, g + it);
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint32_t i = row + u * 64;
-                const bool in = i < s_end;
-                const uint32_t f = res_get(res, (g + it) * U + u);
-                sid[it * U + u] = wa.s.rowids ? wa.s.rowids[in ? i : wa.s_lo] : i;  // wave-uniform test
-                bid[it * U + u] = build_id<IDS>(wa, rid, in && f != 0 ? f - 1 : 0u);
-            }
+        for (int u = 0; u < U; u++) {
+            const uint32_t i = row + u * 64;
+            sid[it * U + u] = wa.s.rowids ? wa.s.rowids[i < wa.s_end ? i : wa.s_lo] : i;  // wave-uniform test
         }
+    }
+}
+
+// Writes the matches probe_walk kept in iterations g .. g + G: each matched
+// row's entry, then (when the build chunk has equal keys) the equal ones
+// further down its chain. The build-side row ids come from LDS.
+template <int G, int PV, typename Tab>
+__device__ __forceinline__ void replay_group(const WalkArgs &wa, const Tab &tab, int g,
+                                             const uint32_t (&res)[ProbeShape<PV>::RES],
+                                             const uint32_t (&sid)[G * ProbeShape<PV>::U], Emitter &em) {
+    constexpr int U = ProbeShape<PV>::U, TH = ProbeShape<PV>::TH;
+    const uint32_t ob1 = wa.ob1;
 #pragma unroll
-        for (int it = 0; it < G; it++) {
-            if (walk_wave_row<U, TH>(wa, g + it) >= s_end) break;  // wave-uniform
+    for (int it = 0; it < G; it++) {
+        if (walk_wave_row<U, TH>(wa, g + it) >= wa.s_end) break;  // wave-uniform
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint32_t f = res_get(res, (g + it) * U + u);
-                const bool m = f != 0;
-                const uint32_t o = m ? f - 1 : 0u;
-                em.put(m, bid[it * U + u] + ob1, sid[it * U + u] + ob1, wa);
-                if (wa.dup) {  // wave-uniform
-                    uint32_t x = m ? nxt[o] : 0u;
-                    while (__ballot(x != 0)) {
-                        const bool has = x != 0;
-                        const uint32_t r = has ? x - 1 : 0u;
-                        em.put(has, (has ? build_id<IDS>(wa, rid, r) : 0u) + ob1, sid[it * U + u] + ob1, wa);
-                        x = has ? nxt[r] : 0u;
-                    }
+        for (int u = 0; u < U; u++) {
+            const uint32_t f = res_get(res, (g + it) * U + u);
+            em.put(f != 0, tab.id[f] + ob1, sid[it * U + u] + ob1, wa);
+            if (wa.dup) {  // wave-uniform
+                uint32_t x = tab.nxt[f];
+                while (__ballot(x != 0)) {
+                    em.put(x != 0 && tab.eq(x, f), tab.id[x] + ob1, sid[it * U + u] + ob1, wa);
+                    x = tab.nxt[x];
                 }
             }
         }
@@ -686,16 +856,18 @@ template <int HP, int KW, int NC, int PV>
 __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * NC, PV>())) void k_probe(PipeArgs a) {
     using KT = typename KeyT<KW>::T;
     constexpr int KB = KW * NC;
-    constexpr int CAP = probe_cap(KB, PV);
+    constexpr int CAP = probe_cap(KB, PV), HEADS = probe_heads(KB, PV);
     constexpr int TH = ProbeShape<PV>::TH, WAVES = ProbeShape<PV>::WAVES;
     extern __shared__ __align__(16) unsigned char smem[];
-    KT *rk = reinterpret_cast<KT *>(smem);                       // [NC][CAP]
-    uint32_t *slots = reinterpret_cast<uint32_t *>(rk + NC * CAP);  // [2 * CAP]
-    uint16_t *nxt = reinterpret_cast<uint16_t *>(slots + 2 * CAP);  // [CAP] chain of equal keys (index + 1, 0: end)
-    constexpr bool IDS = table_keeps_ids(KB);
-    uint32_t *rid = reinterpret_cast<uint32_t *>(nxt + CAP);  // [CAP] build rows' ids (IDS only)
+    using Tab = LdsTable<KT, NC, CAP>;
+    Tab tab;
+    tab.key = reinterpret_cast<KT *>(smem);
+    tab.id = reinterpret_cast<uint32_t *>(tab.key + NC * (CAP + 1));
+    tab.nxt = reinterpret_cast<uint16_t *>(tab.id + CAP + 1);
+    tab.head = reinterpret_cast<uint16_t *>(smem + probe_table_bytes(KB, PV) - 2 * HEADS);
+    uint32_t *head2 = reinterpret_cast<uint32_t *>(tab.head);  // two heads per word
     __shared__ ProbeTask t;
-    uint32_t res[ProbeShape<PV>::RES];  // per probe row its matched build row + 1 (0: none), two per word
+    uint32_t res[ProbeShape<PV>::RES];  // per probe row its first matching entry (0: none), two per word
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     Emitter em;
@@ -703,20 +875,26 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
     const HashCfg hc = a.hash;
     const unsigned long long total = a.ctl->task_total;
 
-    // Lane 0 of wave 0 holds the ticket of the block's next task, fetched
-    // while the current one runs.
-    unsigned long long next_task = ~0ull;
+    // Lane 0 of wave 0 holds the block's next task: block b's first is task b,
+    // the following ones come from the queue (tickets count from the grid
+    // size), fetched while the current one runs; no ticket is drawn when every
+    // task is some block's first. In the wide block, with nothing else on the
+    // CU to cover the set-up, the next task's map entry and partition bounds
+    // are loaded along the way too (`ahead`: they are there).
+    unsigned long long next_task = blockIdx.x, next_pt = 0;
+    uint32_t next_q = 0, next_r0 = 0, next_r1 = 0, next_s0 = 0, next_s1 = 0, ahead = 0;
     if (tid == 0) t.jn = ~0u;  // read and written by this thread only (lane 0 of wave 0)
     while (true) {
         if (w == 0) {
-            unsigned long long task = 0;
-            if (lane == 0) task = next_task != ~0ull ? next_task : atomicAdd(&a.ctl->task_ticket, 1ull);
-            task = __shfl(task, 0, 64);
+            const unsigned long long task = __shfl(next_task, 0, 64);
             if (task >= total) {
                 if (lane == 0) t.done = 1;
             } else {
-                uint32_t jn, q;
-                if (task < a.taskmap_cap) {  // wave-uniform
+                uint32_t jn = 0, q = 0;
+                const bool ready = PV != 0 && uniform(ahead) != 0;
+                if (ready) {
+                    q = next_q;
+                } else if (task < a.taskmap_cap) {  // wave-uniform
                     const unsigned long long e = a.taskmap[task];
                     jn = (uint32_t)(e >> 32);
                     q = (uint32_t)e;
@@ -726,7 +904,7 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
                     q = wave_upper_index(a.ptask + jd0.ptask_off, jd0.nparts, task - a.task0[jn]);
                 }
                 if (lane == 0) {
-                    if (jn != t.jn) {  // a join's fixed fields, kept while its tasks follow each other
+                    if (!ready && jn != t.jn) {  // a join's fixed fields, kept while its tasks follow each other
                         const JoinDesc &jd = a.joins[jn];
                         const JobDesc &jr = a.jobs[jd.job_r];
                         const JobDesc &js = a.jobs[jd.job_s];
@@ -760,20 +938,23 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
                     }
                     // the partition's sides and the task's chunks: one round of loads
                     const uint32_t cap_r = t.cap_r, cap_s = t.cap_s;
-                    const uint32_t r0 = a.base[t.rb + q], s0 = a.base[t.sb + q];
-                    const uint32_t nr = a.base[t.re + q] - r0, ns = a.base[t.se + q] - s0;
+                    if (!ready) {
+                        next_r0 = a.base[t.rb + q], next_s0 = a.base[t.sb + q];
+                        next_r1 = a.base[t.re + q], next_s1 = a.base[t.se + q];
+                        next_pt = t.pt[q];
+                    }
+                    const uint32_t r0 = next_r0, s0 = next_s0, nr = next_r1 - r0, ns = next_s1 - s0;
                     const uint32_t s_chunks = (ns + cap_s - 1) / cap_s;
-                    const uint32_t k = (uint32_t)(task - t.task0 - t.pt[q]);
+                    const uint32_t k = (uint32_t)(task - t.task0 - next_pt);
                     const uint32_t rc = k / s_chunks, sc = k - rc * s_chunks;
                     t.r_lo = r0 + rc * cap_r;
                     t.r_n = nr - rc * cap_r < cap_r ? nr - rc * cap_r : cap_r;
                     t.s_lo = s0 + sc * cap_s;
                     t.s_n = ns - sc * cap_s < cap_s ? ns - sc * cap_s : cap_s;
-                    uint32_t ns2 = 64;
-                    // load <= 1/4 where the slot array (2 * CAP) allows, else <= 1/2:
-                    // a probe round costs the wave's longest chain, not the mean
-                    while (ns2 < 4 * t.r_n && ns2 < 2 * (uint32_t)CAP) ns2 <<= 1;
-                    t.nslots = ns2;
+                    uint32_t nh = 64;  // four heads per row where the table has them, else at least 1.8
+                    while (nh < 4 * t.r_n && nh < (uint32_t)HEADS) nh <<= 1;
+                    t.nheads = nh;
+                    t.hshift = (uint32_t)__builtin_clz(nh) + 1;
                     t.dup = 0;
                     t.done = 0;
                 }
@@ -781,15 +962,27 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
         }
         __syncthreads();
         if (t.done) break;
-        if (w == 0 && lane == 0) next_task = atomicAdd(&a.ctl->task_ticket, 1ull);
+        if (tid == 0) next_task = total > gridDim.x ? gridDim.x + atomicAdd(&a.ctl->task_ticket, 1ull) : total;
+        constexpr int U = ProbeShape<PV>::U, ITERS = ProbeShape<PV>::ITERS;
+        WalkArgs wa;
+        Key<KW, NC> nk[U];
+        if constexpr (PV != 0) {
+            wa = walk_args(t);
+            walk_load<U, TH, KW, NC>(wa, 0, nk);  // crosses the build
+        }
 
-        // build: load the R chunk, then insert (index + 1, 16-bit tag) into buckets;
-        // a key already in the table is chained in front of its entry instead
-        const uint32_t r_lo = t.r_lo, r_n = t.r_n, nslots = t.nslots, bmask = (nslots >> 2) - 1, shift = t.shift;
-        for (uint32_t i = tid; i < nslots; i += TH) slots[i] = 0;
+        // build: load the R chunk, push every row on its chain, look for equal keys
+        const uint32_t r_lo = t.r_lo, r_n = t.r_n, nheads = t.nheads, hshift = t.hshift, shift = t.shift;
+        for (uint32_t i = tid; i < nheads / 2; i += TH) head2[i] = 0;
+        if (tid == 0) {  // entry 0: the end of a chain
+            tab.nxt[0] = 0;
+            tab.id[0] = 0;
+#pragma unroll
+            for (int c = 0; c < NC; c++) tab.key[c * (CAP + 1)] = 0;
+        }
         {
-            // two R rows per lane in flight at once (a task has r_n >= 1)
-            constexpr int RB = 2;
+            // R rows in flight per lane (a task has r_n >= 1)
+            constexpr int RB = PV && KB <= 16 ? 4 : 2;
             const GView rv = uniform_view(t.r);
             for (uint32_t i0 = 0; i0 < r_n; i0 += RB * TH) {
                 Key<KW, NC> rkey[RB];
@@ -799,77 +992,137 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
                     const uint32_t i = i0 + tid + r * TH;
                     const uint32_t row = r_lo + (i < r_n ? i : 0u);
                     rkey[r] = load_key<KW, NC>(rv, row);
-                    if constexpr (IDS) rrow[r] = rv.rowids ? rv.rowids[row] : row;  // wave-uniform test
+                    rrow[r] = rv.rowids ? rv.rowids[row] : row;  // wave-uniform test
                 }
 #pragma unroll
                 for (int r = 0; r < RB; r++) {
                     const uint32_t i = i0 + tid + r * TH;
                     if (i < r_n) {
 #pragma unroll
-                        for (int c = 0; c < NC; c++) rk[c * CAP + i] = rkey[r].c[c];
-                        if constexpr (IDS) rid[i] = rrow[r];
+                        for (int c = 0; c < NC; c++) tab.key[c * (CAP + 1) + i + 1] = rkey[r].c[c];
+                        tab.id[i + 1] = rrow[r];
                     }
                 }
             }
         }
         __syncthreads();
-        for (uint32_t i = tid; i < r_n; i += TH) {
+        // push: the link is written before the compare-and-swap that publishes
+        // the row (a half word swapped through its whole word)
+        for (uint32_t i = tid + 1; i <= r_n; i += TH) {
             Key<KW, NC> k;
 #pragma unroll
-            for (int c = 0; c < NC; c++) k.c[c] = rk[c * CAP + i];
-            const uint32_t place = table_place(hash_key_lo<HP, KW, NC>(k, hc), shift, bmask);  // tag never 0: an entry is never 0
-            const uint32_t tag = place >> 16;
-            const uint32_t e = (tag << 16) | (i + 1);
-            uint32_t b = place & 0xFFFFu;
-            // Scan slots in order (the bucket, then the next buckets). An empty
-            // slot takes the row as a new entry; the entry of an equal key takes
-            // it as its new chain head (nxt[i] = old head). nxt[i] is written
-            // before the CAS that publishes the row, and never changes after.
-            bool placed = false;
-            while (!placed) {
-                for (uint32_t j = 0; j < (uint32_t)kBucketSlots && !placed; j++) {
-                    uint32_t *sl = &slots[b * kBucketSlots + j];
-                    nxt[i] = 0;
-                    uint32_t old = atomicCAS(sl, 0u, e);
-                    placed = old == 0;
-                    while (!placed && (old >> 16) == tag) {
-                        const uint32_t o = (old & 0xFFFFu) - 1;
-                        bool eq = true;
-#pragma unroll
-                        for (int c = 0; c < NC; c++) eq &= rk[c * CAP + o] == k.c[c];
-                        if (!eq) break;  // another key with the same tag: go on scanning
-                        t.dup = 1;
-                        nxt[i] = (uint16_t)(o + 1);
-                        const uint32_t prev = atomicCAS(sl, old, e);
-                        placed = prev == old;
-                        old = prev;  // another row of this key became the head first: chain behind it
-                    }
-                }
-                b = (b + 1) & bmask;
+            for (int c = 0; c < NC; c++) k.c[c] = tab.key[c * (CAP + 1) + i];
+            const uint32_t h = chain_of(hash_key_lo<HP, KW, NC>(k, hc), shift, hshift), sh = (h & 1) * 16;
+            uint32_t old = head2[h >> 1];
+            while (true) {
+                tab.nxt[i] = (uint16_t)(old >> sh);
+                const uint32_t got = atomicCAS(&head2[h >> 1], old, (old & ~(0xFFFFu << sh)) | (i << sh));
+                if (got == old) break;
+                old = got;
             }
+        }
+        __syncthreads();
+        // equal keys in the chunk: whether a row's key comes again further down its chain
+        for (uint32_t i = tid + 1; i <= r_n; i += TH) {
+            uint32_t x = tab.nxt[i];
+            while (x != 0 && !tab.eq(x, i)) x = tab.nxt[x];
+            if (x != 0) t.dup = 1;
         }
         __syncthreads();
 
         // find and count every row's matches (kept in registers), reserve the
-        // task's output rows with one atomic, then write them
-        const WalkArgs wa = walk_args(t);
+        // walk's output rows with one atomic, then write them
+        unsigned long long entry = ~0ull;  // the next task's map entry
+        if constexpr (PV == 0) {
+            wa = walk_args(t);
+            walk_load<U, TH, KW, NC>(wa, 0, nk);
+        }
+        wa.dup = uniform(t.dup) != 0;
+        if (PV != 0 && tid == 0 && next_task < total && next_task < a.taskmap_cap) entry = a.taskmap[next_task];
 #pragma unroll
         for (int k = 0; k < ProbeShape<PV>::RES; k++) res[k] = 0;  // results of skipped iterations read as no match
-        const uint32_t wc = probe_walk<HP, KW, NC, PV>(wa, hc, rk, slots, nxt, res);
-        if (lane == 0) t.wave_count[w] = wc;
-        __syncthreads();
-        if (tid == 0) {
-            uint32_t sum = 0;
-            for (int k = 0; k < WAVES; k++) sum += t.wave_count[k];
-            t.out_base = sum ? atomicAdd(t.count, (unsigned long long)sum) : 0;
-        }
-        __syncthreads();
-        if (wc) {
-            em.pos = t.out_base;
-            for (uint32_t k = 0; k < w; k++) em.pos += t.wave_count[k];
-            // row-id groups of four iterations for single keys of up to 8 bytes (FNV / XOR) and where the
-            // build rows' ids come from LDS (keys wider than 8 bytes; eight in the wide block)
-            replay_walk<(KB <= 8 && HP != HP_GENERIC) ? 4 : (IDS ? (PV ? 8 : 4) : 1), PV, IDS>(wa, nxt, rid, res, em);
+        uint32_t wc = probe_walk<HP, KW, NC, PV>(wa, hc, tab, nk, res);
+        if (lane == 0) t.wave_count[0][w] = wc;
+        if constexpr (PV == 0) {  // a task is one walk
+            __syncthreads();
+            if (tid == 0) {
+                uint32_t sum = 0;
+                for (int k = 0; k < WAVES; k++) sum += t.wave_count[0][k];
+                t.out_base[0] = sum ? atomicAdd(t.count, (unsigned long long)sum) : 0;
+            }
+            __syncthreads();
+            if (wc) {
+                em.pos = t.out_base[0];
+                for (uint32_t k = 0; k < w; k++) em.pos += t.wave_count[0][k];
+                constexpr int G = 4;  // ids loaded four iterations at a time
+                static_assert(ITERS % G == 0, "replay groups");
+#pragma unroll
+                for (int g = 0; g < ITERS; g += G) {
+                    if (walk_wave_row<U, TH>(wa, g) >= wa.s_end) break;  // wave-uniform
+                    uint32_t sid[G * U];
+                    load_ids<G, PV>(wa, g, sid);
+                    replay_group<G, PV>(wa, tab, g, res, sid, em);
+                }
+            }
+        } else {
+            // A task may be several walks (one block per CU: nothing else hides
+            // a walk's reservation or its first loads). While walk k + 1 runs,
+            // the atomic that reserves walk k's rows and the loads of its row
+            // ids are in flight; the first keys of walk k + 2 cross the writing
+            // of walk k. One barrier per walk orders all of it. Four buffers:
+            // a wave may still read walk k's counts while another posts walk
+            // k + 2's.
+            ahead = 0;
+            if (tid == 0 && (uint32_t)(entry >> 32) == t.jn) {
+                next_q = (uint32_t)entry;
+                next_r0 = a.base[t.rb + next_q], next_s0 = a.base[t.sb + next_q];
+                next_r1 = a.base[t.re + next_q], next_s1 = a.base[t.se + next_q];
+                next_pt = t.pt[next_q];
+                ahead = 1;
+            }
+            const uint32_t task_end = uniform(t.s_lo + t.s_n), walks = (uniform(t.s_n) + kProbeChunk - 1) / kProbeChunk;
+            auto advance = [&](WalkArgs &x) {
+                x.s_lo = x.s_end;
+                x.s_end = task_end - x.s_lo < (uint32_t)kProbeChunk ? task_end : x.s_lo + kProbeChunk;
+            };
+            WalkArgs wn = wa;  // the next walk, its first keys in nk
+            if (walks > 1) {
+                advance(wn);
+                walk_load<U, TH, KW, NC>(wn, 0, nk);
+            }
+            __syncthreads();
+            for (uint32_t k = 0; k < walks; k++) {
+                unsigned long long base = 0;
+                if (tid == 0) {
+                    uint32_t sum = 0;
+                    for (int x = 0; x < WAVES; x++) sum += t.wave_count[k & 3][x];
+                    if (sum) base = atomicAdd(t.count, (unsigned long long)sum);
+                }
+                uint32_t done[ProbeShape<PV>::RES], sid[ITERS * U];
+#pragma unroll
+                for (int x = 0; x < ProbeShape<PV>::RES; x++) done[x] = res[x];
+                load_ids<ITERS, PV>(wa, 0, sid);
+                const WalkArgs wd = wa;
+                const uint32_t wcd = wc;
+                if (k + 1 < walks) {
+                    wa = wn;
+#pragma unroll
+                    for (int x = 0; x < ProbeShape<PV>::RES; x++) res[x] = 0;
+                    wc = probe_walk<HP, KW, NC, PV>(wa, hc, tab, nk, res);
+                    if (lane == 0) t.wave_count[(k + 1) & 3][w] = wc;
+                    if (k + 2 < walks) {
+                        advance(wn);
+                        walk_load<U, TH, KW, NC>(wn, 0, nk);
+                    }
+                }
+                if (tid == 0) t.out_base[k & 3] = base;
+                __syncthreads();
+                if (wcd) {
+                    em.pos = t.out_base[k & 3];
+                    for (uint32_t x = 0; x < w; x++) em.pos += t.wave_count[k & 3][x];
+                    replay_group<ITERS, PV>(wd, tab, 0, done, sid, em);
+                }
+            }
         }
         __syncthreads();
     }
@@ -891,8 +1144,11 @@ size_t pass_lds_bytes(int kw, int nc, int tile) {
 }
 
 size_t probe_lds_bytes(int kw, int nc, int table) {
-    const int kb = kw * nc;
-    return (size_t)probe_cap(kb, table) * table_row_bytes(kb);
+    return (size_t)probe_table_bytes(kw * nc, table);
+}
+
+size_t fan_lds_bytes(int kw, int nc, int big, uint32_t bins) {
+    return (size_t)fan_tile(kw * nc, big) * (kw + 2) + (size_t)bins * 8;
 }
 
 }  // namespace
@@ -926,14 +1182,42 @@ template <int HP> hipError_t StageLaunch<HP>::pass(const PipeArgs &a, const Laun
     });
 }
 
+template <int HP> hipError_t StageLaunch<HP>::fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s) {
+    return dispatch_keys(sh, [&]<int KW, int NC>() {
+        hipLaunchKernelGGL((k_fan_hist<HP, KW, NC>), dim3(a.total_hist_blocks), dim3(kFanThreads), (size_t)a.fan_bins * 4, s, a);
+        return hipGetLastError();
+    });
+}
+
+template <int HP> hipError_t StageLaunch<HP>::fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s) {
+    const size_t lds = fan_lds_bytes(sh.kw, sh.nc, sh.fan_big, a.fan_bins);
+    // large tiles: one persistent block per CU; small ones: a block per tile, two at a time per CU
+    const uint32_t cus = sh.cus >= (int)kXcds ? (uint32_t)sh.cus / kXcds * kXcds : kXcds;
+    const dim3 g(sh.fan_big && a.total_p1_tiles > cus ? cus : a.total_p1_tiles);
+    return dispatch_keys(sh, [&]<int KW, int NC>() {
+        if (sh.fan_big)
+            hipLaunchKernelGGL((k_fan<HP, KW, NC, 1>), g, dim3(kFanThreads), lds, s, a);
+        else
+            hipLaunchKernelGGL((k_fan<HP, KW, NC, 0>), g, dim3(kFanThreads), lds, s, a);
+        return hipGetLastError();
+    });
+}
+
 template <int HP> int StageLaunch<HP>::probe_blocks_per_cu(const LaunchShape &sh) {
     const size_t lds = probe_lds_bytes(sh.kw, sh.nc, sh.table);
     int blocks = 1;
     (void)dispatch_keys(sh, [&]<int KW, int NC>() {
         int n = 0;
-        const hipError_t e =
-            sh.table ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_probe<HP, KW, NC, 1>, probe_threads(1), lds)
-                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_probe<HP, KW, NC, 0>, probe_threads(0), lds);
+        hipError_t e;
+        if (sh.table == 2) {
+            if constexpr (KW * NC <= 8)
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_probe<HP, KW, NC, 2>, probe_threads(2), lds);
+            else
+                e = hipErrorInvalidValue;
+        } else {
+            e = sh.table ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_probe<HP, KW, NC, 1>, probe_threads(1), lds)
+                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_probe<HP, KW, NC, 0>, probe_threads(0), lds);
+        }
         if (e == hipSuccess && n > 0) blocks = n;
         return e;
     });
@@ -943,7 +1227,12 @@ template <int HP> int StageLaunch<HP>::probe_blocks_per_cu(const LaunchShape &sh
 template <int HP> hipError_t StageLaunch<HP>::probe(const PipeArgs &a, const LaunchShape &sh, int blocks, hipStream_t s) {
     const size_t lds = probe_lds_bytes(sh.kw, sh.nc, sh.table);
     return dispatch_keys(sh, [&]<int KW, int NC>() {
-        if (sh.table)
+        if (sh.table == 2) {
+            if constexpr (KW * NC <= 8)
+                hipLaunchKernelGGL((k_probe<HP, KW, NC, 2>), dim3(blocks), dim3(probe_threads(2)), lds, s, a);
+            else
+                return hipErrorInvalidValue;
+        } else if (sh.table)
             hipLaunchKernelGGL((k_probe<HP, KW, NC, 1>), dim3(blocks), dim3(probe_threads(1)), lds, s, a);
         else
             hipLaunchKernelGGL((k_probe<HP, KW, NC, 0>), dim3(blocks), dim3(probe_threads(0)), lds, s, a);

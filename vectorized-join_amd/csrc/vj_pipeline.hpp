@@ -28,6 +28,16 @@
 // after the last pass ("fin"). Partition q of a job occupies rows
 // [base[q], base[q+1]) of "fin"; q = d1 * 2^b2 + d2 (pass-1 digit major).
 //
+// One-pass form (the exact layout's default up to kFanBits radix bits in all,
+// whether the plan calls them one pass or two): no mid copy, no tile prefixes.
+// Tile t of the pipeline belongs to group t % kXcds (the XCD its block runs
+// on); k_fan_hist counts every job's rows by (group, partition), k_fan_plan
+// turns the counts into partition bases and, inside each partition, one write
+// cursor per group, and k_fan takes its rows' runs from its group's cursors
+// with one device atomic per (tile, partition). The runs of one group's tiles
+// follow each other in memory, so the lines they share fill up in one XCD's
+// L2; partitions come out back to back, as after two passes.
+//
 // Region layout (2-pass pipelines that ask for it): no histogram and no scans.
 // Every destination is a region of fixed capacity, and blocks reserve their
 // runs in it with one device atomic per digit:
@@ -58,6 +68,10 @@ constexpr int kMaxPassBits = 8;     // digits per pass <= 256
 constexpr int kMaxHistBits = 14;    // 2D histogram in LDS: 2^14 x 4 B = 64 KiB
 constexpr uint32_t kXcds = 8;       // accelerator dies (XCDs) of an MI355X
 constexpr uint32_t kXcdGroup = 32;  // consecutive pass-2 chunks kept on one XCD
+constexpr int kFanBits = 11;        // radix bits one pass can take (k_fan): 2^11 counters in LDS
+constexpr int kFanThreads = 1024;   // one-pass kernels (k_fan_hist, k_fan_plan, k_fan)
+constexpr uint32_t kFanPlanParts = 1u << kFanBits;  // partitions k_fan_plan handles: two per thread
+static_assert(kFanPlanParts == 2 * kFanThreads, "k_fan_plan: two partitions per thread");
 
 // Kernel shapes, chosen per pipeline by the planner or the autotuner.
 //  tile  0: standard pass tile, 512 threads x pass_items rows (6 / 4 / 2 rows by
@@ -73,36 +87,53 @@ __host__ __device__ constexpr int pass_items(int key_bytes, int tile = 0) {
                      : (tile == 2 ? (key_bytes <= 8 ? 8 : (key_bytes <= 16 ? 6 : 4))
                                   : (key_bytes <= 8 ? 6 : (key_bytes <= 16 ? 4 : 2)));
 }
+// Rows per thread of the one-pass kernel k_fan. Large tiles (2^11 partitions)
+// keep a run at a few rows: 12 of 8-byte keys is the largest tile whose keys
+// fit the LDS (one block per CU); below that, 4096-row tiles leave room for
+// two blocks per CU, whose phases overlap.
+__host__ __device__ constexpr int fan_items(int key_bytes, int big) {
+    return !big ? 4 : (key_bytes <= 8 ? 12 : (key_bytes <= 16 ? 8 : 6));
+}
+__host__ __device__ constexpr int fan_tile(int key_bytes, int big) { return kFanThreads * fan_items(key_bytes, big); }
 constexpr int kTileShapes = 3;
 __host__ __device__ constexpr int pass_tile(int key_bytes, int tile = 0) { return kPassThreads * pass_items(key_bytes, tile); }
 __host__ __device__ constexpr int build_cap(int key_bytes) { return key_bytes <= 8 ? 2048 : 1024; }
-// Build rows' ids are kept in LDS next to the table for keys wider than 8
-// bytes (whose tables are small), so duplicate chains are written without a
-// global load per entry; narrower keys read them from the partitioned table.
-__host__ __device__ constexpr bool table_keeps_ids(int key_bytes) { return key_bytes > 8; }
-// LDS bytes per build row of a table: the key, two 4-byte slots, a 2-byte chain
-// link, and the row id where the table keeps it.
-__host__ __device__ constexpr int table_row_bytes(int key_bytes) {
-    return key_bytes + 10 + (table_keeps_ids(key_bytes) ? 4 : 0);
+// The build+probe block's LDS table: per build row its key, its 4-byte row id
+// and a 2-byte link, and a power of two of 2-byte chain heads. Row entries are
+// counted from 1 (entry 0 stands for the end of a chain), hence the + 1.
+__host__ __device__ constexpr int table_bytes(int key_bytes, int cap, int heads) {
+    return ((cap + 1) * (key_bytes + 6) + 15) / 16 * 16 + heads * 2;
 }
-constexpr int kWideTableBytes = 156 * 1024;  // of the 160 KiB of LDS per CU
-// Largest power of two <= 8192 whose table fits kWideTableBytes (row indexes
-// stay below 2^16 - 1, the no-match marker).
+constexpr int kTableBytes = 162 * 1000;  // of the 160 KiB of LDS per CU; the rest holds the task record
+// Largest power of two <= 8192 whose table, with two heads per row, fits.
 __host__ __device__ constexpr int wide_cap(int key_bytes) {
     int c = 8192;
-    while (c > 1024 && c * table_row_bytes(key_bytes) > kWideTableBytes) c >>= 1;
+    while (c > 1024 && table_bytes(key_bytes, c, 2 * c) > kTableBytes) c >>= 1;
     return c;
 }
-__host__ __device__ constexpr int probe_cap(int key_bytes, int table) { return table ? wide_cap(key_bytes) : build_cap(key_bytes); }
+// table 2: the wide block around 8960 rows (keys of up to 8 bytes): what the
+// LDS holds beside 2^14 heads. 2^11 partitions of a 2^24-row build average 8192
+// rows; 8960 leave 8 standard deviations of their spread.
+constexpr int kFullCap = 8960;
+__host__ __device__ constexpr int probe_cap(int key_bytes, int table) {
+    return table == 0 ? build_cap(key_bytes) : (table == 2 ? kFullCap : wide_cap(key_bytes));
+}
+// Chain heads: as many as keep the block's share of the LDS (a quarter of it
+// for standard tables of up to 8-byte keys), two to four per row.
+__host__ __device__ constexpr int probe_heads(int key_bytes, int table) {
+    return table ? 16384 / (key_bytes > 24 ? 2 : (key_bytes > 16 ? 2 : 1)) : (key_bytes <= 4 ? 8192 : 4096);
+}
+__host__ __device__ constexpr int probe_table_bytes(int key_bytes, int table) {
+    return table_bytes(key_bytes, probe_cap(key_bytes, table), probe_heads(key_bytes, table));
+}
 __host__ __device__ constexpr int probe_threads(int table) { return table ? 1024 : 512; }
-constexpr int kProbeChunk = 16384;  // probe rows per build+probe task
-static_assert((kProbeChunk & (kProbeChunk - 1)) == 0 && (build_cap(4) & (build_cap(4) - 1)) == 0 &&
-                  (build_cap(8) & (build_cap(8) - 1)) == 0 && (build_cap(16) & (build_cap(16) - 1)) == 0 &&
-                  (wide_cap(8) & (wide_cap(8) - 1)) == 0 && (wide_cap(12) & (wide_cap(12) - 1)) == 0,
-              "chunk capacities are powers of two (the task counts are shifts)");
-static_assert(wide_cap(4) == 8192 && wide_cap(8) == 8192 && wide_cap(16) == 4096 && wide_cap(32) == 2048 &&
-                  wide_cap(32) * table_row_bytes(32) <= kWideTableBytes,
+constexpr int kProbeChunk = 16384;  // probe rows one walk of the build+probe kernel covers
+static_assert(wide_cap(4) == 8192 && wide_cap(8) == 8192 && wide_cap(16) == 4096 && wide_cap(24) == 4096 && wide_cap(32) == 2048,
               "wide tables");
+static_assert(probe_table_bytes(8, 1) <= kTableBytes && probe_table_bytes(8, 2) <= kTableBytes &&
+                  probe_table_bytes(16, 1) <= kTableBytes && probe_table_bytes(24, 1) <= kTableBytes &&
+                  probe_table_bytes(32, 1) <= kTableBytes,
+              "tables fit the LDS");
 
 struct JobDesc {
     TView in;                 // the caller's table
@@ -127,9 +158,11 @@ struct JobDesc {
     // [base[base_off + q], base[end_off + q]) of fin (exact layout: end_off =
     // base_off + 1; region layout: a second array, both written by k_tasks)
     uint32_t end_off;
-    uint32_t pad_[2];
+    uint32_t groups;          // one-pass form: write-cursor groups (kXcds, or 1 for few tiles)
+    uint32_t pad_;
     uint64_t tilepre_off;     // u32 offset of tilepre [p1_tiles][2^b1] in the count arena
-    uint64_t m1_off;          // u32 offset of m1 [nrow + 1][2^b1] (region layout: counters [2^b1][nseg])
+    uint64_t m1_off;          // u32 offset of m1 [nrow + 1][2^b1] (region layout: counters [2^b1][nseg];
+                              // one-pass form: counts, then cursors [groups][2^(b1+b2)])
     uint64_t m2_off;          // u32 offset of m2 [nrow + 1][2^(b1+b2)] (2-pass jobs; region layout: counters [2^(b1+b2)])
     // Resident build sides. res_base != null: the job is already partitioned
     // (fin_* point at a resident table, res_base at its 2^(b1+b2)+1 bases) and
@@ -143,7 +176,7 @@ struct JoinDesc {
     uint32_t job_r, job_s;
     uint32_t *out_r, *out_s;
     uint64_t cap;             // output capacity (pairs)
-    uint32_t cap_r, cap_s;    // tuples per build chunk / probe chunk (powers of two)
+    uint32_t cap_r, cap_s;    // tuples per build chunk / probe chunk 
     uint32_t ptask_off;       // u64 offset of the per-partition task prefix (nparts + 1)
     uint32_t nparts;          // 2^(b1+b2)
     uint32_t slot_shift;      // hash bits consumed by partitioning (slot uses h >> slot_shift)
@@ -197,6 +230,8 @@ struct PipeArgs {
     uint32_t max_hist_bins;         // LDS bins of the histogram kernel
     uint32_t pass_tile;             // tuples per radix-pass tile (pass_tile(key bytes, tile shape))
     uint32_t regions;               // region layout (every job: two passes, 2^b1 a multiple of kXcds)
+    uint32_t fan_bins;              // one-pass form: partitions of the largest job (0: another form)
+    uint64_t count_words;           // one-pass form: words of the count arena (zeroed before k_fan_hist)
     HashCfg hash;
 };
 
@@ -205,6 +240,7 @@ struct LaunchShape {
     int hp, kw, nc;  // hash path, key width, key columns
     int cus;         // compute units of the device
     int tile, table; // kernel shapes (see pass_items / probe_cap)
+    int fan_big;     // one-pass form: large tiles (see fan_items)
 };
 
 // The hashing stages (histogram, radix pass, build+probe), compiled once per
@@ -213,6 +249,8 @@ struct LaunchShape {
 template <int HP> struct StageLaunch {
     static hipError_t hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
     static hipError_t pass(const PipeArgs &a, const LaunchShape &sh, int pass, hipStream_t s);
+    static hipError_t fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
+    static hipError_t fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
     static hipError_t probe(const PipeArgs &a, const LaunchShape &sh, int blocks, hipStream_t s);
     static int probe_blocks_per_cu(const LaunchShape &sh);
 };
@@ -221,6 +259,10 @@ extern template struct StageLaunch<HP_XOR_HW>;
 extern template struct StageLaunch<HP_GENERIC>;
 hipError_t launch_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_scan(const PipeArgs &a, hipStream_t s);
+hipError_t launch_fan_reset(const PipeArgs &a, hipStream_t s);
+hipError_t launch_fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
+hipError_t launch_fan_plan(const PipeArgs &a, hipStream_t s);
+hipError_t launch_fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_region_reset(const PipeArgs &a, hipStream_t s);
 hipError_t launch_tasks(const PipeArgs &a, hipStream_t s);
 hipError_t launch_reset_probe(const PipeArgs &a, hipStream_t s);
