@@ -224,9 +224,11 @@ template <typename HT> struct Walker {
     }
 
     // One chunk value; V is uint32_t (a word) or signed char (an 8-bit chunk).
-    template <typename V> __device__ __forceinline__ void step(V v) {
+    template <typename V> __device__ __forceinline__ void step(V v) { step_kind(v, kind); }
+    template <int K> __device__ __forceinline__ void step_as(uint32_t v) { step_kind(v, K); }
+    template <typename V> __device__ __forceinline__ void step_kind(V v, int k) {
         typedef HT hash_t;
-        switch (kind) {
+        switch (k) {
         case HK_FNV:  // hash.cu:96-111
             hash ^= v;
             hash *= Fnv<HT>::prime;
@@ -290,6 +292,9 @@ template <typename HT> struct Walker {
 
     __device__ __forceinline__ void chunk_end() {
         if (kind == HK_ADD_HW) hash = bit_reverse<HT>(hash);  // hash.cu:199
+    }
+    template <int K> __device__ __forceinline__ void chunk_end_as() {
+        if (K == HK_ADD_HW) hash = bit_reverse<HT>(hash);
     }
 };
 
