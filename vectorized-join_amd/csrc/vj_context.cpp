@@ -99,9 +99,7 @@ Err ensure(DevBuf &b, size_t bytes, bool slack) {
     if (b.bytes >= bytes) return Err::ok();
     free_buf(b);
     size_t want = align_up(slack ? bytes + bytes / 8 : bytes);
-    if (hipMalloc(&b.p, want) != hipSuccess) {
-        (void)hipGetLastError();
-        b.p = nullptr;
+    if (device_malloc(&b.p, want) != hipSuccess) {
         return Err::make(VJ_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(want) + " bytes failed");
     }
     b.bytes = want;
@@ -262,9 +260,7 @@ vj_built built_as(const vj_table *t, const vj_hash_opts &hash, int P, int b1, in
 
 Err alloc_built(vj_built *b) {
     b->bytes = built_bytes(b->n, b->n_cols, b->key_width, b->b1, b->b2);
-    if (hipMalloc(&b->mem, b->bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        b->mem = nullptr;
+    if (device_malloc(&b->mem, b->bytes) != hipSuccess) {
         return Err::make(VJ_ERR_OUT_OF_MEMORY, "hipMalloc of a resident table failed");
     }
     char *p = static_cast<char *>(b->mem);
@@ -1102,9 +1098,14 @@ Err set_device(vj_ctx *c) {
     return Err::ok();
 }
 
+// An output column of n row ids; without a budget it may be a kept buffer.
+hipError_t alloc_ids(const vj_ctx *c, uint32_t **p, uint64_t n) {
+    return cache_malloc(reinterpret_cast<void **>(p), n * 4, c->budget == 0);
+}
+
 // Runs the pipeline for `specs`; counts[i] receives join i's match count.
 // When `grow` is set, joins whose output overflowed get a fresh buffer of the
-// exact size (hipMalloc, owned by the caller) and only build+probe is rerun.
+// exact size (alloc_ids, owned by the caller) and only build+probe is rerun.
 // Graph use of a pipeline: never, always (vj_join_batch with use_graph), or
 // automatically when the same launch signature comes twice in a row.
 enum GraphMode { GRAPH_OFF, GRAPH_ON, GRAPH_AUTO };
@@ -1177,12 +1178,11 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
         bool again = false;
         for (size_t i = 0; i < specs.size(); i++) {
             if (counts[i] > specs[i].cap) {
-                if (specs[i].out_r) (void)hipFree(specs[i].out_r);
-                if (specs[i].out_s) (void)hipFree(specs[i].out_s);
+                cache_free(specs[i].out_r, true);  // (the pipeline has ended)
+                cache_free(specs[i].out_s, true);
                 specs[i].out_r = specs[i].out_s = nullptr;
-                if (hipMalloc(&specs[i].out_r, counts[i] * 4) != hipSuccess ||
-                    hipMalloc(&specs[i].out_s, counts[i] * 4) != hipSuccess) {
-                    (void)hipGetLastError();
+                if (alloc_ids(c, &specs[i].out_r, counts[i]) != hipSuccess ||
+                    alloc_ids(c, &specs[i].out_s, counts[i]) != hipSuccess) {
                     return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
                 }
                 specs[i].cap = counts[i];
@@ -1222,16 +1222,15 @@ Err join_callee_alloc(vj_ctx *c, const vj_table *build, const vj_table *probe, c
     if (c->budget && cap * 8 + held_extra > c->budget)  // the output alone breaks the budget: nothing is allocated
         return Err::make(VJ_ERR_BUDGET, "an output of " + std::to_string(cap) + " pairs exceeds the HBM budget");
     std::vector<JoinSpec> specs{{build, probe, nullptr, nullptr, cap}};
-    if (hipMalloc(&specs[0].out_r, cap * 4) != hipSuccess || hipMalloc(&specs[0].out_s, cap * 4) != hipSuccess) {
-        (void)hipGetLastError();
-        if (specs[0].out_r) (void)hipFree(specs[0].out_r);
+    if (alloc_ids(c, &specs[0].out_r, cap) != hipSuccess || alloc_ids(c, &specs[0].out_s, cap) != hipSuccess) {
+        cache_free(specs[0].out_r, true);
         return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
     }
     std::vector<uint64_t> counts;
     const Err e = run_joins(c, specs, opts, s, counts, true, cap * 8 + held_extra, nullptr);
     if (e.failed()) {
-        if (specs[0].out_r) (void)hipFree(specs[0].out_r);
-        if (specs[0].out_s) (void)hipFree(specs[0].out_s);
+        cache_free(specs[0].out_r, false);
+        cache_free(specs[0].out_s, false);
         return e;
     }
     out->count = counts[0];
@@ -1320,6 +1319,7 @@ vj_status vj_ctx_create(int device, vj_ctx **out) {
         c->na_stage = nullptr;
         c->na_error = "hipHostMalloc of the staging block failed";
     }
+    cache_context(device, 1);
     *out = c;
     return VJ_OK;
 }
@@ -1335,6 +1335,7 @@ vj_status vj_ctx_destroy(vj_ctx *c) {
     if (c->na_stage) (void)hipHostFree(c->na_stage);
     for (int i = 0; i < EV_COUNT; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
+    cache_context(c->device, -1);
     delete c;
     return VJ_OK;
 }
@@ -1499,8 +1500,7 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
     if (tmp_words) {
         if (c->budget && held_bytes(c) + tmp_words * 8 > c->budget)
             return fail(c, Err::make(VJ_ERR_BUDGET, "the transposed key columns exceed the HBM budget"));
-        if (hipMalloc(&tmp, tmp_words * 8) != hipSuccess) {
-            (void)hipGetLastError();
+        if (cache_malloc(reinterpret_cast<void **>(&tmp), tmp_words * 8, c->budget == 0) != hipSuccess) {
             return fail(c, Err::make(VJ_ERR_OUT_OF_MEMORY, "hipMalloc of the transposed key columns failed"));
         }
         e = launch_rows_to_cols(r->column_values, r->n_rows, nc, tmp, st, c->cus);
@@ -1522,9 +1522,8 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
     if (!e.failed() && m) {  // rs: (r pk, s pk) per pair, row-major, and primary keys 1..M
         if (c->budget && held_bytes(c) + tmp_words * 8 + m * 8 + m * 24 > c->budget) {
             e = Err::make(VJ_ERR_BUDGET, "the joined table exceeds the HBM budget");
-        } else if (hipMalloc(&rs->column_values, m * 16) != hipSuccess ||
-                   hipMalloc(&rs->primary_keys, m * 8) != hipSuccess) {
-            (void)hipGetLastError();
+        } else if (cache_malloc(reinterpret_cast<void **>(&rs->column_values), m * 16, c->budget == 0) != hipSuccess ||
+                   cache_malloc(reinterpret_cast<void **>(&rs->primary_keys), m * 8, c->budget == 0) != hipSuccess) {
             e = Err::make(VJ_ERR_OUT_OF_MEMORY, "hipMalloc of the joined table failed");
         } else {
             e = launch_materialize(pairs.build_rowids, pairs.probe_rowids, m, r->primary_keys, s->primary_keys,
@@ -1537,8 +1536,9 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
     } else {
         (void)hipStreamSynchronize(st);  // nothing queued may still use what is freed below
     }
-    (void)vj_pairs_free(&pairs);
-    if (tmp) (void)hipFree(tmp);
+    cache_free(pairs.build_rowids, true);
+    cache_free(pairs.probe_rowids, true);
+    cache_free(tmp, true);
     if (e.failed()) {
         (void)vj_rows_free(rs);
         return fail(c, e);
@@ -1550,8 +1550,8 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
 
 vj_status vj_rows_free(vj_rows *t) {
     if (!t) return VJ_ERR_INVALID_ARGUMENT;
-    if (t->column_values) (void)hipFree(t->column_values);
-    if (t->primary_keys) (void)hipFree(t->primary_keys);
+    cache_free(t->column_values, false);
+    cache_free(t->primary_keys, t->column_values != nullptr);  // (the device was waited for just now)
     t->column_values = t->primary_keys = nullptr;
     t->n_rows = 0;
     return VJ_OK;
@@ -1559,8 +1559,8 @@ vj_status vj_rows_free(vj_rows *t) {
 
 vj_status vj_pairs_free(vj_pairs *p) {
     if (!p) return VJ_ERR_INVALID_ARGUMENT;
-    if (p->build_rowids) (void)hipFree(p->build_rowids);
-    if (p->probe_rowids) (void)hipFree(p->probe_rowids);
+    cache_free(p->build_rowids, false);
+    cache_free(p->probe_rowids, p->build_rowids != nullptr);  // (the device was waited for just now)
     p->build_rowids = p->probe_rowids = nullptr;
     p->count = 0;
     return VJ_OK;
@@ -1836,8 +1836,8 @@ vj_status vj_tune(vj_ctx *c, const vj_table *build, const vj_table *probe, const
     if (e.failed()) return fail(c, e);
     const uint64_t cap = std::max<uint64_t>(counts[0], 1);
     uint32_t *ob = nullptr, *op = nullptr;
-    if (hipMalloc(&ob, cap * 4) != hipSuccess || hipMalloc(&op, cap * 4) != hipSuccess) {
-        (void)hipGetLastError();
+    if (device_malloc(reinterpret_cast<void **>(&ob), cap * 4) != hipSuccess ||
+        device_malloc(reinterpret_cast<void **>(&op), cap * 4) != hipSuccess) {
         if (ob) (void)hipFree(ob);
         return fail(c, Err::make(VJ_ERR_OUT_OF_MEMORY, "tuning output allocation failed"));
     }

@@ -52,6 +52,20 @@ Err launch_materialize(const uint32_t *ri, const uint32_t *si, uint64_t m, const
 
 int device_cu_count(int device);
 
+// vj_cache.cpp: device buffers kept between calls.
+// hipMalloc that gives the kept buffers of the current device back before it
+// reports a failure (nullptr and the error then).
+hipError_t device_malloc(void **p, size_t bytes);
+// A buffer of at least `bytes` on the current device; `keep`: it may come from
+// and go back to the kept ones (false: a plain device_malloc).
+hipError_t cache_malloc(void **p, size_t bytes, bool keep);
+// Takes a buffer back. `idle`: no queued work uses it; else the device is
+// waited for, as hipFree does.
+void cache_free(void *p, bool idle);
+// A context on `device` begins (+1) or ends (-1); the last one's end gives the
+// device's kept buffers back.
+void cache_context(int device, int delta);
+
 // vj_noalloc.hip: the fixed device scratch of vj_join_into_noalloc.
 constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;  // per device, held until the process ends
 static_assert(kNoAllocScratchBytes == VJ_NOALLOC_SCRATCH_BYTES, "the header states the scratch size");
