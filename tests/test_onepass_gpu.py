@@ -118,3 +118,31 @@ def test_kept_and_resident_tables_use_their_own_bits(budget):
         built.free()
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("kw,nc,kind", [(4, 1, "fnv"), (8, 1, "custom_xor_hw"), (4, 3, "custom_add"), (8, 4, "fnv")])
+@pytest.mark.parametrize("nr,ns,dup", [(1, 1, 1), (1, 5000, 1), (1536, 1025, 3), (1537, 40000, 1), (700, 200001, 700)])
+def test_one_launch_form(ctx, kw, nc, kind, nr, ns, dup):
+    """A build side that fits one table: row ids, 1-based output, an output too small and then regrown, calls in a
+    row (its counters start from zero each time); per-stage timing takes the pipeline instead."""
+    import torch
+    rng = np.random.default_rng(nr + ns)
+    r, s = _keys(rng, nr, ns, kw, nc, dup)
+    rid, sid = rng.permutation(nr).astype(np.uint32) + 7, rng.permutation(ns).astype(np.uint32) + 9
+    want = np_join(workloads.reference_rows(r), workloads.reference_rows(s), rid, sid)
+    want = (want[0] + 1, want[1] + 1)
+    m = len(want[0])
+    dr, ds = workloads.to_device(r), workloads.to_device(s)
+    drid, dsid = workloads.to_device([rid])[0], workloads.to_device([sid])[0]
+    opts = vjoin.join_opts(kind, one_based=True)
+    for timed in (False, False, True, False):
+        ctx.set_profiling(timed)
+        got = _pairs(ctx, dr, ds, opts, m, drid, dsid)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    if m > 1:
+        o = [torch.full((m,), -1, dtype=torch.int32, device="cuda") for _ in range(2)]
+        rc, n = ctx.join_into(vjoin.table(dr, drid), vjoin.table(ds, dsid), opts, o[0], o[1], capacity=m - 1)
+        assert vjoin.STATUS[rc] == "VJ_ERR_CAPACITY" and n == m and int(o[0][m - 1]) == -1 == int(o[1][m - 1])
+    a, b = ctx.join(vjoin.table(dr, drid), vjoin.table(ds, dsid), vjoin.join_opts(kind, one_based=True, out_capacity_hint=1))
+    got = sorted_pairs(a.cpu().numpy().view(np.uint32), b.cpu().numpy().view(np.uint32))
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])

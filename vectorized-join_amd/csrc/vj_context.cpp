@@ -67,6 +67,7 @@ struct vj_ctx {
     // creation, so the entry point itself allocates nothing)
     void *na_scratch = nullptr;
     void *na_stage = nullptr;
+    void *direct = nullptr;  // k_direct's counters (zero between joins); null: that form is off
     std::string na_error;
 };
 
@@ -195,7 +196,7 @@ int need_bits(uint64_t nr, int cap) {
 int fan_bits(uint64_t nr, int kb, int table, double share = 1.0) {
     const uint64_t target = (uint64_t)probe_cap(kb, table) * 3 / 4;
     int need = nr > target ? ceil_log2((nr + target - 1) / target) : 0;
-    if (table && nr > target) need = std::max(need, std::min(ceil_log2((uint64_t)(512 * share)), ceil_log2(nr / 256)));
+    if (table && nr > target) need = std::max(need, std::min(ceil_log2((uint64_t)(512 * share)), ceil_log2(nr / 128)));
     return need > kFanBits && table == 1 && kb <= 8 && nr <= (uint64_t)8300 << kFanBits ? kFanBits : need;
 }
 
@@ -885,7 +886,12 @@ PipeArgs make_args(const Arenas &ar, const Plan &pl) {
     a.max_hist_bins = pl.max_hist_bins;
     a.pass_tile = pass_tile(pl.kb, pl.shape.tile);
     a.regions = pl.regions ? 1u : 0u;
+    a.down = reinterpret_cast<unsigned long long *>(ar.pinned + pl.off_count);
+    a.down_words = (uint32_t)(pl.down_bytes() / 8);
     if (pl.fan) {
+        a.up_dst = reinterpret_cast<unsigned long long *>(m);
+        a.up_src = reinterpret_cast<const unsigned long long *>(ar.pinned);
+        a.up_words = (uint32_t)(pl.upload_bytes / 8);
         a.pass_tile = fan_tile(pl.kb, pl.shape.fan_big);
         a.fan_bins = pl.fan_bins;
         a.count_words = pl.counts_words;
@@ -904,8 +910,10 @@ void stage_descriptors(char *h, const Plan &pl) {
     memcpy(h + pl.off_pc0, pl.p2_chunk0.data(), pl.p2_chunk0.size() * 4);
 }
 
+// (In the one-pass form the pipeline's first kernel fetches them from there.)
 Err upload(const Arenas &ar, const Plan &pl, hipStream_t s) {
     stage_descriptors(ar.pinned, pl);
+    if (pl.fan) return Err::ok();
     VJ_HIP_TRY(hipMemcpyAsync(ar.meta, ar.pinned, pl.upload_bytes, hipMemcpyHostToDevice, s));
     return Err::ok();
 }
@@ -916,6 +924,20 @@ Err upload(const Arenas &ar, const Plan &pl, hipStream_t s) {
         if (e_ != hipSuccess)                                                                 \
             return Err::make(VJ_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));  \
     } while (0)
+
+// Blocks of the build+probe launch: what fits the device, but in the one-pass
+// form no more than there are tasks where nothing is skewed (a block without
+// one costs its start and its end).
+int probe_grid(const vj_ctx *c, const Plan &pl) {
+    const uint64_t fit = (uint64_t)c->cus * (uint64_t)probe_blocks_per_cu(pl.shape);
+    if (!pl.fan) return (int)fit;
+    uint64_t tasks = 0;
+    for (const JoinDesc &jd : pl.joins) {
+        const uint64_t nr = pl.jobs[jd.job_r].n, ns = pl.jobs[jd.job_s].n;
+        tasks += (jd.nparts + ns / jd.cap_s) * (nr / jd.nparts / jd.cap_r + 1);
+    }
+    return (int)std::max<uint64_t>(1, std::min(tasks, fit));
+}
 
 // Launches every stage on `s` (no host synchronisation). `events`: record
 // the start / end events (and the per-stage ones when profiling); off while
@@ -934,7 +956,7 @@ Err launch_stages(vj_ctx *c, const Plan &pl, const PipeArgs &a, hipStream_t s, b
         if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_P2], s));
         VJ_LAUNCH(launch_tasks(a, s));
     } else if (pl.fan) {
-        VJ_LAUNCH(launch_fan_reset(a, s));
+        VJ_LAUNCH(launch_fan_begin(a, s));
         VJ_LAUNCH(launch_fan_hist(a, pl.shape, s));
         if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_HIST], s));
         VJ_LAUNCH(launch_fan_plan(a, s));
@@ -953,7 +975,7 @@ Err launch_stages(vj_ctx *c, const Plan &pl, const PipeArgs &a, hipStream_t s, b
         if (prof) VJ_HIP_TRY(hipEventRecord(c->ev[EV_P2], s));
     }
     if (with_probe && !pl.joins.empty())
-        VJ_LAUNCH(launch_probe(a, pl.shape, c->cus * probe_blocks_per_cu(pl.shape), s));
+        VJ_LAUNCH(launch_probe(a, pl.shape, probe_grid(c, pl), s));
     if (events) VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
     return Err::ok();
 }
@@ -968,7 +990,7 @@ std::vector<uint64_t> graph_signature(const vj_ctx *c, const Plan &pl, const Pip
            (uint64_t)pl.shape.fan_big << 4;
     x[1] = (uint64_t)pl.shape.hp | (uint64_t)pl.shape.kw << 8 | (uint64_t)pl.shape.nc << 16 |
            (uint64_t)pl.shape.tile << 24 | (uint64_t)pl.shape.table << 32;
-    x[2] = (uint64_t)c->cus * (uint64_t)probe_blocks_per_cu(pl.shape);
+    x[2] = (uint64_t)probe_grid(c, pl);
     x[3] = pl.upload_bytes;
     x[4] = pl.off_count;
     x[5] = pl.joins.size();
@@ -985,10 +1007,11 @@ void drop_graph(vj_ctx *c) {
     c->graph_sig.clear();
 }
 
-// Captures upload -> all stages -> count download on the context's capture
-// stream (capture needs a stream other than the null stream) and instantiates
-// it. The upload and the download are kernels that read / write the pinned
-// staging buffer (no copy nodes: a replay stays on the compute queue). Events
+// Captures upload -> all stages on the context's capture stream (capture needs
+// a stream other than the null stream) and instantiates it. The upload is a
+// kernel that reads the pinned staging buffer, and the build+probe kernel
+// writes the counts to it (no copy nodes: a replay stays on the compute
+// queue). Events
 // are recorded around the graph launch, not inside the graph (event nodes
 // inside a replayed graph gave stage times that did not add up).
 Err capture_pipeline(vj_ctx *c, const Plan &pl, const PipeArgs &a) {
@@ -997,13 +1020,9 @@ Err capture_pipeline(vj_ctx *c, const Plan &pl, const PipeArgs &a) {
     hipStream_t cs = c->capture_stream;
     char *h = static_cast<char *>(c->pinned);
     VJ_HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeRelaxed));
-    hipError_t he = launch_stage_copy(c->meta.p, h, pl.upload_bytes, cs);
+    hipError_t he = pl.fan ? hipSuccess : launch_stage_copy(c->meta.p, h, pl.upload_bytes, cs);
     Err e = he == hipSuccess ? launch_stages(c, pl, a, cs, true, false)
                              : Err::make(VJ_ERR_HIP, std::string("capture upload: ") + hipGetErrorString(he));
-    if (!e.failed()) {
-        he = launch_stage_copy(h + pl.off_count, static_cast<char *>(c->meta.p) + pl.off_count, pl.down_bytes(), cs);
-        if (he != hipSuccess) e = Err::make(VJ_ERR_HIP, std::string("capture download: ") + hipGetErrorString(he));
-    }
     hipGraph_t g = nullptr;
     he = hipStreamEndCapture(cs, &g);
     if (!e.failed() && he != hipSuccess) e = Err::make(VJ_ERR_HIP, std::string("end capture: ") + hipGetErrorString(he));
@@ -1103,6 +1122,54 @@ hipError_t alloc_ids(const vj_ctx *c, uint32_t **p, uint64_t n) {
     return cache_malloc(reinterpret_cast<void **>(p), n * 4, c->budget == 0);
 }
 
+// Whether a plan runs as one launch (k_direct): a single join without
+// partitions whose build side fits one table. Under a budget and with
+// per-stage timing the pipeline runs as ever.
+bool may_run_direct(const vj_ctx *c, const Plan &pl) {
+    if (!pl.fan || pl.joins.size() != 1 || pl.any_part || c->budget || c->profiling || !c->direct || !c->na_stage) return false;
+    const JobDesc &r = pl.jobs[pl.joins[0].job_r], &s = pl.jobs[pl.joins[0].job_s];
+    return !r.b1 && !s.b1 && r.n > 0 && s.n > 0 && r.n <= pl.joins[0].cap_r;
+}
+
+Err run_direct(vj_ctx *c, Plan &pl, JoinSpec &js, hipStream_t s, std::vector<uint64_t> &counts, bool grow, int *retries_out) {
+    const JoinDesc &jd = pl.joins[0];
+    unsigned long long *down = static_cast<unsigned long long *>(c->na_stage);
+    DirectArgs d;
+    memset(&d, 0, sizeof(d));
+    d.r = pl.jobs[jd.job_r].in;
+    d.s = pl.jobs[jd.job_s].in;
+    d.cap_s = jd.cap_s;
+    d.one_based = jd.one_based;
+    d.count = static_cast<unsigned long long *>(c->direct);
+    d.done = d.count + 32;  // on another line
+    d.down = down;
+    d.hash = pl.hash;
+    const int blocks = (int)((d.s.n + d.cap_s - 1) / d.cap_s);
+    int retries = 0;
+    while (true) {
+        d.out_r = js.out_r;
+        d.out_s = js.out_s;
+        d.cap = js.cap;
+        VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
+        VJ_LAUNCH(launch_direct(d, pl.shape, blocks, s));
+        VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
+        VJ_HIP_TRY(hipStreamSynchronize(s));
+        if (!grow || down[0] <= js.cap) break;
+        const uint64_t m = down[0];
+        cache_free(js.out_r, true);
+        cache_free(js.out_s, true);
+        js.out_r = js.out_s = nullptr;
+        if (alloc_ids(c, &js.out_r, m) != hipSuccess || alloc_ids(c, &js.out_s, m) != hipSuccess)
+            return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
+        js.cap = m;
+        retries = 1;
+    }
+    counts.assign(1, down[0]);
+    if (retries_out) *retries_out = retries;
+    fill_summary(c, pl, js, counts[0], (uint64_t)blocks, retries, false, held_bytes(c));
+    return Err::ok();
+}
+
 // Runs the pipeline for `specs`; counts[i] receives join i's match count.
 // When `grow` is set, joins whose output overflowed get a fresh buffer of the
 // exact size (alloc_ids, owned by the caller) and only build+probe is rerun.
@@ -1115,6 +1182,7 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
               GraphMode gmode = GRAPH_OFF) {
     Plan pl;
     VJ_TRY(plan_joins(pl, specs, o, c, true, c->budget != 0));
+    if (may_run_direct(c, pl)) return run_direct(c, pl, specs[0], s, counts, grow, retries_out);
     VJ_TRY(admit(c, pl, extra_bytes + pl.keep_bytes));
     VJ_TRY(allocate(c, pl));
     PipeArgs a = make_args(ctx_arenas(c), pl);
@@ -1151,8 +1219,6 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
     } else {
         VJ_TRY(upload(ctx_arenas(c), pl, s));
         VJ_TRY(launch_stages(c, pl, a, s, true));
-        VJ_HIP_TRY(hipMemcpyAsync(hc, static_cast<char *>(c->meta.p) + pl.off_count, pl.down_bytes(),
-                                  hipMemcpyDeviceToHost, s));
     }
     VJ_HIP_TRY(hipStreamSynchronize(s));
     if (pl.regions && reinterpret_cast<const Ctl *>(h + pl.off_ctl)->overflow) {
@@ -1198,10 +1264,8 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
             VJ_HIP_TRY(hipMemcpyAsync(static_cast<char *>(c->meta.p) + pl.off_joins, h + pl.off_joins,
                                       pl.joins.size() * sizeof(JoinDesc), hipMemcpyHostToDevice, s));
             VJ_LAUNCH(launch_reset_probe(a, s));
-            VJ_LAUNCH(launch_probe(a, pl.shape, c->cus * probe_blocks_per_cu(pl.shape), s));
+            VJ_LAUNCH(launch_probe(a, pl.shape, probe_grid(c, pl), s));
             VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
-            VJ_HIP_TRY(hipMemcpyAsync(hc, static_cast<char *>(c->meta.p) + pl.off_count, pl.down_bytes(),
-                                      hipMemcpyDeviceToHost, s));
             VJ_HIP_TRY(hipStreamSynchronize(s));
             counts.assign(hc, hc + pl.joins.size());
         }
@@ -1263,9 +1327,6 @@ Err pipeline_launch(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts 
     VJ_TRY(upload(ctx_arenas(c), pl, s));
     PipeArgs a = make_args(ctx_arenas(c), pl);
     VJ_TRY(launch_stages(c, pl, a, s, true));
-    char *h = static_cast<char *>(c->pinned);
-    VJ_HIP_TRY(hipMemcpyAsync(h + pl.off_count, static_cast<char *>(c->meta.p) + pl.off_count, pl.down_bytes(),
-                              hipMemcpyDeviceToHost, s));
     *count_off = pl.off_count;
     return Err::ok();
 }
@@ -1319,6 +1380,13 @@ vj_status vj_ctx_create(int device, vj_ctx **out) {
         c->na_stage = nullptr;
         c->na_error = "hipHostMalloc of the staging block failed";
     }
+    // counters of the one-launch form (without them joins take the pipeline)
+    if (hipMalloc(&c->direct, 512) != hipSuccess || hipMemset(c->direct, 0, 512) != hipSuccess ||
+        hipDeviceSynchronize() != hipSuccess) {
+        (void)hipGetLastError();
+        if (c->direct) (void)hipFree(c->direct);
+        c->direct = nullptr;
+    }
     cache_context(device, 1);
     *out = c;
     return VJ_OK;
@@ -1333,6 +1401,7 @@ vj_status vj_ctx_destroy(vj_ctx *c) {
     free_all(c);
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->na_stage) (void)hipHostFree(c->na_stage);
+    if (c->direct) (void)hipFree(c->direct);
     for (int i = 0; i < EV_COUNT; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     cache_context(c->device, -1);
@@ -1440,9 +1509,7 @@ vj_status vj_join_into_noalloc(vj_ctx *c, const vj_table *build, const vj_table 
     e = upload(ar, pl, s);
     if (!e.failed()) e = launch_stages(c, pl, a, s, true);
     if (!e.failed()) {
-        hipError_t he = hipMemcpyAsync(ar.pinned + pl.off_count, ar.meta + pl.off_count, pl.down_bytes(),
-                                       hipMemcpyDeviceToHost, s);
-        if (he == hipSuccess) he = hipStreamSynchronize(s);
+        const hipError_t he = hipStreamSynchronize(s);
         if (he != hipSuccess) e = Err::make(VJ_ERR_HIP, std::string("no-allocation join: ") + hipGetErrorString(he));
     }
     if (e.failed()) return fail(c, e);

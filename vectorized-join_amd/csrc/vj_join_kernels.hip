@@ -34,6 +34,8 @@
 // This file holds the scan kernels and the launchers; the hashing stages
 // (k_hist, k_pass, k_probe) are in vj_join_stages.hpp, compiled once per hash
 // path (vj_join_fnv.hip, vj_join_xorhw.hip, vj_join_generic.hip).
+#include <algorithm>
+
 #include "vj_kernel_common.hpp"
 
 namespace vj {
@@ -170,6 +172,7 @@ __global__ __launch_bounds__(1024) void k_bases(PipeArgs a) {
         if (threadIdx.x == 0) {
             a.ctl->task_ticket = 0;
             a.ctl->overflow = 0;
+            a.ctl->done = 0;
         }
         for (uint32_t j = threadIdx.x; j < a.n_joins; j += blockDim.x) a.out_count[j] = 0;
     }
@@ -355,14 +358,16 @@ __global__ __launch_bounds__(1024) void k_task_offsets(PipeArgs a) {
     }
 }
 
-// One-pass form, before the histogram: zeroes the count arena, the queue
-// ticket and the output counters.
-__global__ __launch_bounds__(1024) void k_fan_reset(PipeArgs a) {
+// One-pass form, before the histogram: fetches the descriptors from the host's
+// staging buffer, zeroes the count arena, the queue ticket and the output counters.
+__global__ __launch_bounds__(1024) void k_fan_begin(PipeArgs a) {
     const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
     if (i0 == 0) {
         a.ctl->task_ticket = 0;
         a.ctl->overflow = 0;
+        a.ctl->done = 0;
     }
+    for (uint32_t i = i0; i < a.up_words; i += step) a.up_dst[i] = a.up_src[i];
     const gptr<uint32_t> c = to_global(a.counts);
     for (uint64_t i = i0; i < a.count_words; i += step) c[i] = 0;
     for (uint32_t j = i0; j < a.n_joins; j += step) a.out_count[j] = 0;
@@ -483,6 +488,7 @@ __global__ __launch_bounds__(1024) void k_region_reset(PipeArgs a) {
         if (threadIdx.x == 0) {
             a.ctl->task_ticket = 0;
             a.ctl->overflow = 0;
+            a.ctl->done = 0;
         }
         for (uint32_t j = threadIdx.x; j < a.n_joins; j += blockDim.x) a.out_count[j] = 0;
     }
@@ -567,9 +573,18 @@ hipError_t launch_region_reset(const PipeArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_fan_reset(const PipeArgs &a, hipStream_t s) {
-    const uint64_t blocks = (a.count_words + 4095) / 4096;
-    hipLaunchKernelGGL(k_fan_reset, dim3((unsigned)(blocks < 1 ? 1 : (blocks < 512 ? blocks : 512))), dim3(1024), 0, s, a);
+hipError_t launch_direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s) {
+    switch (sh.hp) {
+    case HP_FNV: return StageLaunch<HP_FNV>::direct(d, sh, blocks, s);
+    case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::direct(d, sh, blocks, s);
+    case HP_GENERIC: return StageLaunch<HP_GENERIC>::direct(d, sh, blocks, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_fan_begin(const PipeArgs &a, hipStream_t s) {
+    const uint64_t blocks = std::max<uint64_t>((a.count_words + 4095) / 4096, (a.up_words + 1023) / 1024);
+    hipLaunchKernelGGL(k_fan_begin, dim3((unsigned)(blocks < 1 ? 1 : (blocks < 512 ? blocks : 512))), dim3(1024), 0, s, a);
     return hipGetLastError();
 }
 

@@ -851,27 +851,255 @@ template <int HP, int KB, int PV> constexpr int probe_waves_per_simd() {
     return PV ? 4 : (KB <= 8 && HP != HP_GENERIC ? 8 : 4);
 }
 
-// PV: table shape (probe_cap, probe_threads).
-template <int HP, int KW, int NC, int PV>
-__global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * NC, PV>())) void k_probe(PipeArgs a) {
+// The block's table in its dynamic LDS.
+template <int KW, int NC, int PV>
+__device__ __forceinline__ LdsTable<typename KeyT<KW>::T, NC, probe_cap(KW * NC, PV)> lds_table(unsigned char *smem) {
     using KT = typename KeyT<KW>::T;
-    constexpr int KB = KW * NC;
-    constexpr int CAP = probe_cap(KB, PV), HEADS = probe_heads(KB, PV);
-    constexpr int TH = ProbeShape<PV>::TH, WAVES = ProbeShape<PV>::WAVES;
-    extern __shared__ __align__(16) unsigned char smem[];
-    using Tab = LdsTable<KT, NC, CAP>;
-    Tab tab;
+    constexpr int CAP = probe_cap(KW * NC, PV);
+    LdsTable<KT, NC, CAP> tab;
     tab.key = reinterpret_cast<KT *>(smem);
     tab.id = reinterpret_cast<uint32_t *>(tab.key + NC * (CAP + 1));
     tab.nxt = reinterpret_cast<uint16_t *>(tab.id + CAP + 1);
-    tab.head = reinterpret_cast<uint16_t *>(smem + probe_table_bytes(KB, PV) - 2 * HEADS);
-    uint32_t *head2 = reinterpret_cast<uint32_t *>(tab.head);  // two heads per word
-    __shared__ ProbeTask t;
-    uint32_t res[ProbeShape<PV>::RES];  // per probe row its first matching entry (0: none), two per word
+    tab.head = reinterpret_cast<uint16_t *>(smem + probe_table_bytes(KW * NC, PV) - 2 * probe_heads(KW * NC, PV));
+    return tab;
+}
 
+// Chain heads of a task's table: four per row where the table has them, else at least 1.8.
+__device__ __forceinline__ void set_heads(ProbeTask &t, uint32_t most) {
+    uint32_t nh = 64;
+    while (nh < 4 * t.r_n && nh < most) nh <<= 1;
+    t.nheads = nh;
+    t.hshift = (uint32_t)__builtin_clz(nh) + 1;
+}
+
+// Builds the table of task t's build chunk and joins its probe rows with it
+// (block-wide; the record is complete). The caller's hooks run between the
+// phases: after_build before the first walk, after_walk after it (wide block).
+template <int HP, int KW, int NC, int PV, typename Build, typename Walk>
+__device__ __forceinline__ void run_task(ProbeTask &t, const HashCfg &hc, unsigned char *smem, Build after_build, Walk after_walk) {
+    constexpr int KB = KW * NC, CAP = probe_cap(KB, PV);
+    constexpr int TH = ProbeShape<PV>::TH, WAVES = ProbeShape<PV>::WAVES;
+    const auto tab = lds_table<KW, NC, PV>(smem);
+    uint32_t *head2 = reinterpret_cast<uint32_t *>(tab.head);  // two heads per word
+    uint32_t res[ProbeShape<PV>::RES];  // per probe row its first matching entry (0: none), two per word
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     Emitter em;
     em.pos = 0;
+            constexpr int U = ProbeShape<PV>::U, ITERS = ProbeShape<PV>::ITERS;
+            WalkArgs wa;
+            Key<KW, NC> nk[U];
+            if constexpr (PV != 0) {
+                wa = walk_args(t);
+                walk_load<U, TH, KW, NC>(wa, 0, nk);  // crosses the build
+            }
+
+            // build: load the R chunk, push every row on its chain, look for equal keys
+            const uint32_t r_lo = t.r_lo, r_n = t.r_n, nheads = t.nheads, hshift = t.hshift, shift = t.shift;
+            for (uint32_t i = tid; i < nheads / 2; i += TH) head2[i] = 0;
+            if (tid == 0) {  // entry 0: the end of a chain
+                tab.nxt[0] = 0;
+                tab.id[0] = 0;
+#pragma unroll
+                for (int c = 0; c < NC; c++) tab.key[c * (CAP + 1)] = 0;
+            }
+            {
+                // R rows in flight per lane (a task has r_n >= 1)
+                constexpr int RB = PV && KB <= 16 ? 4 : 2;
+                const GView rv = uniform_view(t.r);
+                for (uint32_t i0 = 0; i0 < r_n; i0 += RB * TH) {
+                    Key<KW, NC> rkey[RB];
+                    uint32_t rrow[RB];
+#pragma unroll
+                    for (int r = 0; r < RB; r++) {
+                        const uint32_t i = i0 + tid + r * TH;
+                        const uint32_t row = r_lo + (i < r_n ? i : 0u);
+                        rkey[r] = load_key<KW, NC>(rv, row);
+                        rrow[r] = rv.rowids ? rv.rowids[row] : row;  // wave-uniform test
+                    }
+#pragma unroll
+                    for (int r = 0; r < RB; r++) {
+                        const uint32_t i = i0 + tid + r * TH;
+                        if (i < r_n) {
+#pragma unroll
+                            for (int c = 0; c < NC; c++) tab.key[c * (CAP + 1) + i + 1] = rkey[r].c[c];
+                            tab.id[i + 1] = rrow[r];
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            // push: the link is written before the compare-and-swap that publishes
+            // the row (a half word swapped through its whole word)
+            for (uint32_t i = tid + 1; i <= r_n; i += TH) {
+                Key<KW, NC> k;
+#pragma unroll
+                for (int c = 0; c < NC; c++) k.c[c] = tab.key[c * (CAP + 1) + i];
+                const uint32_t h = chain_of(hash_key_lo<HP, KW, NC>(k, hc), shift, hshift), sh = (h & 1) * 16;
+                uint32_t old = head2[h >> 1];
+                while (true) {
+                    tab.nxt[i] = (uint16_t)(old >> sh);
+                    const uint32_t got = atomicCAS(&head2[h >> 1], old, (old & ~(0xFFFFu << sh)) | (i << sh));
+                    if (got == old) break;
+                    old = got;
+                }
+            }
+            __syncthreads();
+            // equal keys in the chunk: whether a row's key comes again further down its chain
+            for (uint32_t i = tid + 1; i <= r_n; i += TH) {
+                uint32_t x = tab.nxt[i];
+                while (x != 0 && !tab.eq(x, i)) x = tab.nxt[x];
+                if (x != 0) t.dup = 1;
+            }
+            __syncthreads();
+
+            // find and count every row's matches (kept in registers), reserve the
+            // walk's output rows with one atomic, then write them
+            if constexpr (PV == 0) {
+                wa = walk_args(t);
+                walk_load<U, TH, KW, NC>(wa, 0, nk);
+            }
+            wa.dup = uniform(t.dup) != 0;
+            after_build();
+#pragma unroll
+            for (int k = 0; k < ProbeShape<PV>::RES; k++) res[k] = 0;  // results of skipped iterations read as no match
+            uint32_t wc = probe_walk<HP, KW, NC, PV>(wa, hc, tab, nk, res);
+            if (lane == 0) t.wave_count[0][w] = wc;
+            if constexpr (PV == 0) {  // a task is one walk
+                __syncthreads();
+                if (tid == 0) {
+                    uint32_t sum = 0;
+                    for (int k = 0; k < WAVES; k++) sum += t.wave_count[0][k];
+                    t.out_base[0] = sum ? atomicAdd(t.count, (unsigned long long)sum) : 0;
+                }
+                __syncthreads();
+                if (wc) {
+                    em.pos = t.out_base[0];
+                    for (uint32_t k = 0; k < w; k++) em.pos += t.wave_count[0][k];
+                    constexpr int G = 4;  // ids loaded four iterations at a time
+                    static_assert(ITERS % G == 0, "replay groups");
+#pragma unroll
+                    for (int g = 0; g < ITERS; g += G) {
+                        if (walk_wave_row<U, TH>(wa, g) >= wa.s_end) break;  // wave-uniform
+                        uint32_t sid[G * U];
+                        load_ids<G, PV>(wa, g, sid);
+                        replay_group<G, PV>(wa, tab, g, res, sid, em);
+                    }
+                }
+            } else {
+                // A task may be several walks (one block per CU: nothing else hides
+                // a walk's reservation or its first loads). While walk k + 1 runs,
+                // the atomic that reserves walk k's rows and the loads of its row
+                // ids are in flight; the first keys of walk k + 2 cross the writing
+                // of walk k. One barrier per walk orders all of it. Four buffers:
+                // a wave may still read walk k's counts while another posts walk
+                // k + 2's.
+                after_walk();
+                const uint32_t task_end = uniform(t.s_lo + t.s_n), walks = (uniform(t.s_n) + kProbeChunk - 1) / kProbeChunk;
+                auto advance = [&](WalkArgs &x) {
+                    x.s_lo = x.s_end;
+                    x.s_end = task_end - x.s_lo < (uint32_t)kProbeChunk ? task_end : x.s_lo + kProbeChunk;
+                };
+                WalkArgs wn = wa;  // the next walk, its first keys in nk
+                if (walks > 1) {
+                    advance(wn);
+                    walk_load<U, TH, KW, NC>(wn, 0, nk);
+                }
+                __syncthreads();
+                for (uint32_t k = 0; k < walks; k++) {
+                    unsigned long long base = 0;
+                    if (tid == 0) {
+                        uint32_t sum = 0;
+                        for (int x = 0; x < WAVES; x++) sum += t.wave_count[k & 3][x];
+                        if (sum) base = atomicAdd(t.count, (unsigned long long)sum);
+                    }
+                    uint32_t done[ProbeShape<PV>::RES], sid[ITERS * U];
+#pragma unroll
+                    for (int x = 0; x < ProbeShape<PV>::RES; x++) done[x] = res[x];
+                    load_ids<ITERS, PV>(wa, 0, sid);
+                    const WalkArgs wd = wa;
+                    const uint32_t wcd = wc;
+                    if (k + 1 < walks) {
+                        wa = wn;
+#pragma unroll
+                        for (int x = 0; x < ProbeShape<PV>::RES; x++) res[x] = 0;
+                        wc = probe_walk<HP, KW, NC, PV>(wa, hc, tab, nk, res);
+                        if (lane == 0) t.wave_count[(k + 1) & 3][w] = wc;
+                        if (k + 2 < walks) {
+                            advance(wn);
+                            walk_load<U, TH, KW, NC>(wn, 0, nk);
+                        }
+                    }
+                    if (tid == 0) t.out_base[k & 3] = base;
+                    __syncthreads();
+                    if (wcd) {
+                        em.pos = t.out_base[k & 3];
+                        for (uint32_t x = 0; x < w; x++) em.pos += t.wave_count[k & 3][x];
+                        replay_group<ITERS, PV>(wd, tab, 0, done, sid, em);
+                    }
+                }
+            }
+    __syncthreads();
+}
+
+// Ends a block: the last one of the grid copies the counters (and what stands
+// behind them, `words` in all) to the host's buffer, so that no copy has to
+// follow the kernel, and clears the block count for the next launch. Only
+// atomics touch the counters while blocks run, and this thread has the results
+// of its own before it counts the block: no fence is needed (one writes the
+// L2 back, in every block: 8-12 us of a 60 us launch).
+__device__ __forceinline__ bool finish_block(uint32_t &flag, unsigned long long *done, unsigned long long *src,
+                                             unsigned long long *dst, uint32_t words) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        flag = atomicAdd(done, 1ull) + 1 == gridDim.x;
+    }
+    __syncthreads();
+    if (!flag) return false;
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x)
+        dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) *done = 0;
+    return true;
+}
+
+// One join without partitions whose build side fits a table: one launch, the
+// tables by value, no descriptors in memory, a block per probe chunk. Each
+// block builds the whole table; up to some thousand rows that is cheaper than
+// any partitioning (2^10 x 2^13 rows: 33 us of device work in five launches
+// before, one launch now).
+template <int HP, int KW, int NC, int PV>
+__global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * NC, PV>())) void k_direct(DirectArgs d) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ ProbeTask t;
+    if (threadIdx.x == 0) {
+        t.r = d.r;
+        t.s = d.s;
+        t.out_r = d.out_r;
+        t.out_s = d.out_s;
+        t.count = d.count;
+        t.cap = d.cap;
+        t.r_lo = 0;
+        t.r_n = (uint32_t)d.r.n;
+        t.s_lo = blockIdx.x * d.cap_s;
+        t.s_n = (uint32_t)d.s.n - t.s_lo < d.cap_s ? (uint32_t)d.s.n - t.s_lo : d.cap_s;
+        t.shift = 0;
+        t.one_based = d.one_based;
+        t.dup = 0;
+        set_heads(t, (uint32_t)probe_heads(KW * NC, PV));
+    }
+    __syncthreads();
+    run_task<HP, KW, NC, PV>(t, d.hash, smem, [] {}, [] {});
+    if (finish_block(t.done, d.done, d.count, d.down, 1)) {
+        __syncthreads();
+        if (threadIdx.x == 0) *d.count = 0;  // for the next join
+    }
+}
+
+// PV: table shape (probe_cap, probe_threads).
+template <int HP, int KW, int NC, int PV>
+__global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * NC, PV>())) void k_probe(PipeArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ ProbeTask t;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const HashCfg hc = a.hash;
     const unsigned long long total = a.ctl->task_total;
 
@@ -951,10 +1179,7 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
                     t.r_n = nr - rc * cap_r < cap_r ? nr - rc * cap_r : cap_r;
                     t.s_lo = s0 + sc * cap_s;
                     t.s_n = ns - sc * cap_s < cap_s ? ns - sc * cap_s : cap_s;
-                    uint32_t nh = 64;  // four heads per row where the table has them, else at least 1.8
-                    while (nh < 4 * t.r_n && nh < (uint32_t)HEADS) nh <<= 1;
-                    t.nheads = nh;
-                    t.hshift = (uint32_t)__builtin_clz(nh) + 1;
+                    set_heads(t, (uint32_t)probe_heads(KW * NC, PV));
                     t.dup = 0;
                     t.done = 0;
                 }
@@ -963,169 +1188,24 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
         __syncthreads();
         if (t.done) break;
         if (tid == 0) next_task = total > gridDim.x ? gridDim.x + atomicAdd(&a.ctl->task_ticket, 1ull) : total;
-        constexpr int U = ProbeShape<PV>::U, ITERS = ProbeShape<PV>::ITERS;
-        WalkArgs wa;
-        Key<KW, NC> nk[U];
-        if constexpr (PV != 0) {
-            wa = walk_args(t);
-            walk_load<U, TH, KW, NC>(wa, 0, nk);  // crosses the build
-        }
-
-        // build: load the R chunk, push every row on its chain, look for equal keys
-        const uint32_t r_lo = t.r_lo, r_n = t.r_n, nheads = t.nheads, hshift = t.hshift, shift = t.shift;
-        for (uint32_t i = tid; i < nheads / 2; i += TH) head2[i] = 0;
-        if (tid == 0) {  // entry 0: the end of a chain
-            tab.nxt[0] = 0;
-            tab.id[0] = 0;
-#pragma unroll
-            for (int c = 0; c < NC; c++) tab.key[c * (CAP + 1)] = 0;
-        }
-        {
-            // R rows in flight per lane (a task has r_n >= 1)
-            constexpr int RB = PV && KB <= 16 ? 4 : 2;
-            const GView rv = uniform_view(t.r);
-            for (uint32_t i0 = 0; i0 < r_n; i0 += RB * TH) {
-                Key<KW, NC> rkey[RB];
-                uint32_t rrow[RB];
-#pragma unroll
-                for (int r = 0; r < RB; r++) {
-                    const uint32_t i = i0 + tid + r * TH;
-                    const uint32_t row = r_lo + (i < r_n ? i : 0u);
-                    rkey[r] = load_key<KW, NC>(rv, row);
-                    rrow[r] = rv.rowids ? rv.rowids[row] : row;  // wave-uniform test
-                }
-#pragma unroll
-                for (int r = 0; r < RB; r++) {
-                    const uint32_t i = i0 + tid + r * TH;
-                    if (i < r_n) {
-#pragma unroll
-                        for (int c = 0; c < NC; c++) tab.key[c * (CAP + 1) + i + 1] = rkey[r].c[c];
-                        tab.id[i + 1] = rrow[r];
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        // push: the link is written before the compare-and-swap that publishes
-        // the row (a half word swapped through its whole word)
-        for (uint32_t i = tid + 1; i <= r_n; i += TH) {
-            Key<KW, NC> k;
-#pragma unroll
-            for (int c = 0; c < NC; c++) k.c[c] = tab.key[c * (CAP + 1) + i];
-            const uint32_t h = chain_of(hash_key_lo<HP, KW, NC>(k, hc), shift, hshift), sh = (h & 1) * 16;
-            uint32_t old = head2[h >> 1];
-            while (true) {
-                tab.nxt[i] = (uint16_t)(old >> sh);
-                const uint32_t got = atomicCAS(&head2[h >> 1], old, (old & ~(0xFFFFu << sh)) | (i << sh));
-                if (got == old) break;
-                old = got;
-            }
-        }
-        __syncthreads();
-        // equal keys in the chunk: whether a row's key comes again further down its chain
-        for (uint32_t i = tid + 1; i <= r_n; i += TH) {
-            uint32_t x = tab.nxt[i];
-            while (x != 0 && !tab.eq(x, i)) x = tab.nxt[x];
-            if (x != 0) t.dup = 1;
-        }
-        __syncthreads();
-
-        // find and count every row's matches (kept in registers), reserve the
-        // walk's output rows with one atomic, then write them
         unsigned long long entry = ~0ull;  // the next task's map entry
-        if constexpr (PV == 0) {
-            wa = walk_args(t);
-            walk_load<U, TH, KW, NC>(wa, 0, nk);
-        }
-        wa.dup = uniform(t.dup) != 0;
-        if (PV != 0 && tid == 0 && next_task < total && next_task < a.taskmap_cap) entry = a.taskmap[next_task];
-#pragma unroll
-        for (int k = 0; k < ProbeShape<PV>::RES; k++) res[k] = 0;  // results of skipped iterations read as no match
-        uint32_t wc = probe_walk<HP, KW, NC, PV>(wa, hc, tab, nk, res);
-        if (lane == 0) t.wave_count[0][w] = wc;
-        if constexpr (PV == 0) {  // a task is one walk
-            __syncthreads();
-            if (tid == 0) {
-                uint32_t sum = 0;
-                for (int k = 0; k < WAVES; k++) sum += t.wave_count[0][k];
-                t.out_base[0] = sum ? atomicAdd(t.count, (unsigned long long)sum) : 0;
-            }
-            __syncthreads();
-            if (wc) {
-                em.pos = t.out_base[0];
-                for (uint32_t k = 0; k < w; k++) em.pos += t.wave_count[0][k];
-                constexpr int G = 4;  // ids loaded four iterations at a time
-                static_assert(ITERS % G == 0, "replay groups");
-#pragma unroll
-                for (int g = 0; g < ITERS; g += G) {
-                    if (walk_wave_row<U, TH>(wa, g) >= wa.s_end) break;  // wave-uniform
-                    uint32_t sid[G * U];
-                    load_ids<G, PV>(wa, g, sid);
-                    replay_group<G, PV>(wa, tab, g, res, sid, em);
+        run_task<HP, KW, NC, PV>(
+            t, hc, smem,
+            [&] {
+                if (PV != 0 && tid == 0 && next_task < total && next_task < a.taskmap_cap) entry = a.taskmap[next_task];
+            },
+            [&] {
+                ahead = 0;
+                if (tid == 0 && (uint32_t)(entry >> 32) == t.jn) {
+                    next_q = (uint32_t)entry;
+                    next_r0 = a.base[t.rb + next_q], next_s0 = a.base[t.sb + next_q];
+                    next_r1 = a.base[t.re + next_q], next_s1 = a.base[t.se + next_q];
+                    next_pt = t.pt[next_q];
+                    ahead = 1;
                 }
-            }
-        } else {
-            // A task may be several walks (one block per CU: nothing else hides
-            // a walk's reservation or its first loads). While walk k + 1 runs,
-            // the atomic that reserves walk k's rows and the loads of its row
-            // ids are in flight; the first keys of walk k + 2 cross the writing
-            // of walk k. One barrier per walk orders all of it. Four buffers:
-            // a wave may still read walk k's counts while another posts walk
-            // k + 2's.
-            ahead = 0;
-            if (tid == 0 && (uint32_t)(entry >> 32) == t.jn) {
-                next_q = (uint32_t)entry;
-                next_r0 = a.base[t.rb + next_q], next_s0 = a.base[t.sb + next_q];
-                next_r1 = a.base[t.re + next_q], next_s1 = a.base[t.se + next_q];
-                next_pt = t.pt[next_q];
-                ahead = 1;
-            }
-            const uint32_t task_end = uniform(t.s_lo + t.s_n), walks = (uniform(t.s_n) + kProbeChunk - 1) / kProbeChunk;
-            auto advance = [&](WalkArgs &x) {
-                x.s_lo = x.s_end;
-                x.s_end = task_end - x.s_lo < (uint32_t)kProbeChunk ? task_end : x.s_lo + kProbeChunk;
-            };
-            WalkArgs wn = wa;  // the next walk, its first keys in nk
-            if (walks > 1) {
-                advance(wn);
-                walk_load<U, TH, KW, NC>(wn, 0, nk);
-            }
-            __syncthreads();
-            for (uint32_t k = 0; k < walks; k++) {
-                unsigned long long base = 0;
-                if (tid == 0) {
-                    uint32_t sum = 0;
-                    for (int x = 0; x < WAVES; x++) sum += t.wave_count[k & 3][x];
-                    if (sum) base = atomicAdd(t.count, (unsigned long long)sum);
-                }
-                uint32_t done[ProbeShape<PV>::RES], sid[ITERS * U];
-#pragma unroll
-                for (int x = 0; x < ProbeShape<PV>::RES; x++) done[x] = res[x];
-                load_ids<ITERS, PV>(wa, 0, sid);
-                const WalkArgs wd = wa;
-                const uint32_t wcd = wc;
-                if (k + 1 < walks) {
-                    wa = wn;
-#pragma unroll
-                    for (int x = 0; x < ProbeShape<PV>::RES; x++) res[x] = 0;
-                    wc = probe_walk<HP, KW, NC, PV>(wa, hc, tab, nk, res);
-                    if (lane == 0) t.wave_count[(k + 1) & 3][w] = wc;
-                    if (k + 2 < walks) {
-                        advance(wn);
-                        walk_load<U, TH, KW, NC>(wn, 0, nk);
-                    }
-                }
-                if (tid == 0) t.out_base[k & 3] = base;
-                __syncthreads();
-                if (wcd) {
-                    em.pos = t.out_base[k & 3];
-                    for (uint32_t x = 0; x < w; x++) em.pos += t.wave_count[k & 3][x];
-                    replay_group<ITERS, PV>(wd, tab, 0, done, sid, em);
-                }
-            }
-        }
-        __syncthreads();
+            });
     }
+    (void)finish_block(t.done, &a.ctl->done, a.out_count, a.down, a.down_words);
 }
 
 // Dispatch over the key shape (key width, key columns).
@@ -1222,6 +1302,17 @@ template <int HP> int StageLaunch<HP>::probe_blocks_per_cu(const LaunchShape &sh
         return e;
     });
     return blocks > 8 ? 8 : blocks;
+}
+
+template <int HP> hipError_t StageLaunch<HP>::direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s) {
+    const size_t lds = probe_lds_bytes(sh.kw, sh.nc, sh.table);
+    return dispatch_keys(sh, [&]<int KW, int NC>() {
+        if (sh.table)
+            hipLaunchKernelGGL((k_direct<HP, KW, NC, 1>), dim3(blocks), dim3(probe_threads(1)), lds, s, d);
+        else
+            hipLaunchKernelGGL((k_direct<HP, KW, NC, 0>), dim3(blocks), dim3(probe_threads(0)), lds, s, d);
+        return hipGetLastError();
+    });
 }
 
 template <int HP> hipError_t StageLaunch<HP>::probe(const PipeArgs &a, const LaunchShape &sh, int blocks, hipStream_t s) {

@@ -201,10 +201,12 @@ struct ColScanDesc {
 // layout), the total written by k_tasks (one join) or k_scan2, before the
 // build+probe kernel reads them. overflow: a region of the region layout
 // received more rows than it holds (set by k_tasks).
+// done: build+probe blocks that have ended; the last one sets it back to 0.
 struct Ctl {
     unsigned long long task_ticket;
     unsigned long long task_total;
     unsigned long long overflow;
+    unsigned long long done;
 };
 
 
@@ -232,6 +234,25 @@ struct PipeArgs {
     uint32_t regions;               // region layout (every job: two passes, 2^b1 a multiple of kXcds)
     uint32_t fan_bins;              // one-pass form: partitions of the largest job (0: another form)
     uint64_t count_words;           // one-pass form: words of the count arena (zeroed before k_fan_hist)
+    // one-pass form: the descriptors' way from the host's staging buffer, in words of 8 bytes
+    unsigned long long *up_dst;
+    const unsigned long long *up_src;
+    uint32_t up_words;
+    // out_count and what follows it (to the end of ctl) goes to the host's buffer when build+probe ends
+    uint32_t down_words;
+    unsigned long long *down;
+    HashCfg hash;
+};
+
+// One join without partitions (k_direct). count and done are zero before the
+// launch and after it; the match count is written to `down` (host memory).
+struct DirectArgs {
+    TView r, s;
+    uint32_t *out_r, *out_s;
+    uint64_t cap;
+    uint32_t cap_s;  // probe rows per block
+    uint32_t one_based;
+    unsigned long long *count, *done, *down;
     HashCfg hash;
 };
 
@@ -252,6 +273,7 @@ template <int HP> struct StageLaunch {
     static hipError_t fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
     static hipError_t fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
     static hipError_t probe(const PipeArgs &a, const LaunchShape &sh, int blocks, hipStream_t s);
+    static hipError_t direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s);
     static int probe_blocks_per_cu(const LaunchShape &sh);
 };
 extern template struct StageLaunch<HP_FNV>;
@@ -259,7 +281,8 @@ extern template struct StageLaunch<HP_XOR_HW>;
 extern template struct StageLaunch<HP_GENERIC>;
 hipError_t launch_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_scan(const PipeArgs &a, hipStream_t s);
-hipError_t launch_fan_reset(const PipeArgs &a, hipStream_t s);
+hipError_t launch_direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s);
+hipError_t launch_fan_begin(const PipeArgs &a, hipStream_t s);
 hipError_t launch_fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_fan_plan(const PipeArgs &a, hipStream_t s);
 hipError_t launch_fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
