@@ -67,6 +67,9 @@ struct vj_ctx {
     // creation, so the entry point itself allocates nothing)
     void *na_scratch = nullptr;
     void *na_stage = nullptr;
+    // size classes whose build side had chains too long for the flat form: joins
+    // of the class that still skip it
+    std::unordered_map<uint64_t, int> flat_skip;
     void *direct = nullptr;  // k_direct's counters (zero between joins); null: that form is off
     std::string na_error;
 };
@@ -1117,9 +1120,22 @@ Err set_device(vj_ctx *c) {
     return Err::ok();
 }
 
+
 // An output column of n row ids; without a budget it may be a kept buffer.
 hipError_t alloc_ids(const vj_ctx *c, uint32_t **p, uint64_t n) {
     return cache_malloc(reinterpret_cast<void **>(p), n * 4, c->budget == 0);
+}
+
+// A fresh output of m pairs for a callee-allocated join that has more than its
+// first one held (nothing uses that any more).
+Err regrow(const vj_ctx *c, JoinSpec &js, uint64_t m) {
+    cache_free(js.out_r, true);
+    cache_free(js.out_s, true);
+    js.out_r = js.out_s = nullptr;
+    if (alloc_ids(c, &js.out_r, m) != hipSuccess || alloc_ids(c, &js.out_s, m) != hipSuccess)
+        return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
+    js.cap = m;
+    return Err::ok();
 }
 
 // Whether a plan runs as one launch (k_direct): a single join without
@@ -1129,6 +1145,100 @@ bool may_run_direct(const vj_ctx *c, const Plan &pl) {
     if (!pl.fan || pl.joins.size() != 1 || pl.any_part || c->budget || c->profiling || !c->direct || !c->na_stage) return false;
     const JobDesc &r = pl.jobs[pl.joins[0].job_r], &s = pl.jobs[pl.joins[0].job_s];
     return !r.b1 && !s.b1 && r.n > 0 && s.n > 0 && r.n <= pl.joins[0].cap_r;
+}
+
+// Whether a join runs in the flat form: a single planner-driven join (no
+// plan of the caller's or the tuner's) whose build side is past an LDS table
+// and whose table an XCD's L2 holds. Under a budget and with per-stage timing
+// the pipeline runs as ever.
+bool may_run_flat(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_opts *o) {
+    if (c->budget || c->profiling || !c->direct || !c->na_stage || specs.size() != 1 || specs[0].res || specs[0].keep) return false;
+    if (o->passes != -1 || o->bits1 || o->bits2 || o->tile || o->table || o->layout == VJ_LAYOUT_REGIONS) return false;
+    const vj_table *r = specs[0].r, *s = specs[0].s;
+    const int kb = s->key_width * s->n_cols;
+    if (r->n_rows <= (uint64_t)build_cap(kb) * 3 / 4 || r->n_rows > flat_max_rows(kb) || s->n_rows == 0) return false;
+    HashCfg h;
+    if (make_hash_cfg(&o->hash, s, &h).failed()) return false;
+    const uint64_t key = tune_key(r->n_rows, kb, hash_path(h));
+    if (c->tuned.count(key)) return false;
+    auto it = c->flat_skip.find(key);
+    if (it == c->flat_skip.end()) return true;
+    if (--it->second <= 0) c->flat_skip.erase(it);
+    return false;
+}
+
+// *ran: false if the build side has more equal keys than the form follows; the
+// join then runs in the pipeline, and so do the next ones of its size class.
+Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std::vector<uint64_t> &counts, bool grow,
+             int *retries_out, bool *ran) {
+    *ran = true;
+    VJ_TRY(check_pair(js.r, js.s));
+    FlatArgs a;
+    memset(&a, 0, sizeof(a));
+    VJ_TRY(make_hash_cfg(&o->hash, js.s, &a.hash));
+    a.r = to_view(js.r);
+    a.s = to_view(js.s);
+    LaunchShape sh{};
+    sh.hp = hash_path(a.hash);
+    sh.kw = js.s->key_width;
+    sh.nc = js.s->n_cols;
+    sh.cus = c->cus;
+    const int kb = sh.kw * sh.nc;
+    // a quarter full where that still fits, else up to half
+    uint64_t slots = 1ull << ceil_log2(2 * a.r.n);
+    if (slots * 2 * flat_slot_bytes(kb) <= kFlatTableBytes) slots *= 2;
+    const size_t table = slots * flat_slot_bytes(kb), links = align_up(a.r.n * 4);
+    VJ_TRY(ensure(c->tuples, table + kAlign + links, true));
+    char *m = static_cast<char *>(c->tuples.p);
+    a.slots = reinterpret_cast<uint32_t *>(m);
+    a.dup = reinterpret_cast<uint32_t *>(m + table);
+    a.nxt = reinterpret_cast<uint32_t *>(m + table + kAlign);
+    a.mask = (uint32_t)(slots - 1);
+    a.hshift = 32u - (uint32_t)ceil_log2(kb <= 4 ? slots / 2 : slots);
+    a.zero_words = (uint32_t)((table + 16) / 16);
+    a.one_based = o->one_based ? 1 : 0;
+    a.count = static_cast<unsigned long long *>(c->direct);
+    a.done = a.count + 32;
+    a.down = static_cast<unsigned long long *>(c->na_stage);
+    int retries = 0;
+    while (true) {
+        a.out_r = js.out_r;
+        a.out_s = js.out_s;
+        a.cap = js.cap;
+        VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
+        VJ_LAUNCH(launch_flat(a, sh, s));
+        VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
+        VJ_HIP_TRY(hipStreamSynchronize(s));
+        if (a.down[0] & kFlatGiveUp) {
+            c->flat_skip[tune_key(a.r.n, kb, sh.hp)] = 64;
+            *ran = false;
+            return Err::ok();
+        }
+        if (!grow || a.down[0] <= js.cap) break;
+        VJ_TRY(regrow(c, js, a.down[0]));
+        retries = 1;
+    }
+    counts.assign(1, a.down[0]);
+    if (retries_out) *retries_out = retries;
+    vj_join_summary &sm = c->summary;
+    memset(&sm, 0, sizeof(sm));
+    sm.build_rows = a.r.n;
+    sm.probe_rows = a.s.n;
+    sm.matches = counts[0];
+    sm.retries = retries;
+    sm.partitions = 1;
+    sm.tasks = 1;
+    sm.ms_total = elapsed(c->ev[EV_START], c->ev[EV_PROBE]);
+    sm.scratch_bytes = held_bytes(c);
+    sm.tile_rows = pass_tile(kb, 0);
+    sm.probe_threads = kFlatThreads;
+    sm.table_rows = (int32_t)a.r.n;
+    sm.layout = VJ_LAYOUT_EXACT;
+    sm.bytes_build_probe = a.r.n * (kb + (a.r.rowids ? 4u : 0u)) + a.s.n * (kb + (a.s.rowids ? 4u : 0u)) + counts[0] * 8;
+    sm.bytes_total = sm.bytes_build_probe;
+    sm.gbps_total = gbps(sm.bytes_total, sm.ms_total);
+    sm.probe_tuples_per_s = sm.ms_total > 0 ? (double)sm.probe_rows / (sm.ms_total * 1e-3) : 0.0;
+    return Err::ok();
 }
 
 Err run_direct(vj_ctx *c, Plan &pl, JoinSpec &js, hipStream_t s, std::vector<uint64_t> &counts, bool grow, int *retries_out) {
@@ -1155,13 +1265,7 @@ Err run_direct(vj_ctx *c, Plan &pl, JoinSpec &js, hipStream_t s, std::vector<uin
         VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
         VJ_HIP_TRY(hipStreamSynchronize(s));
         if (!grow || down[0] <= js.cap) break;
-        const uint64_t m = down[0];
-        cache_free(js.out_r, true);
-        cache_free(js.out_s, true);
-        js.out_r = js.out_s = nullptr;
-        if (alloc_ids(c, &js.out_r, m) != hipSuccess || alloc_ids(c, &js.out_s, m) != hipSuccess)
-            return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
-        js.cap = m;
+        VJ_TRY(regrow(c, js, down[0]));
         retries = 1;
     }
     counts.assign(1, down[0]);
@@ -1180,6 +1284,11 @@ enum GraphMode { GRAPH_OFF, GRAPH_ON, GRAPH_AUTO };
 Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hipStream_t s,
               std::vector<uint64_t> &counts, bool grow, uint64_t extra_bytes, int *retries_out,
               GraphMode gmode = GRAPH_OFF) {
+    if (may_run_flat(c, specs, o)) {
+        bool ran = false;
+        VJ_TRY(run_flat(c, specs[0], o, s, counts, grow, retries_out, &ran));
+        if (ran) return Err::ok();
+    }
     Plan pl;
     VJ_TRY(plan_joins(pl, specs, o, c, true, c->budget != 0));
     if (may_run_direct(c, pl)) return run_direct(c, pl, specs[0], s, counts, grow, retries_out);
@@ -1244,14 +1353,7 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
         bool again = false;
         for (size_t i = 0; i < specs.size(); i++) {
             if (counts[i] > specs[i].cap) {
-                cache_free(specs[i].out_r, true);  // (the pipeline has ended)
-                cache_free(specs[i].out_s, true);
-                specs[i].out_r = specs[i].out_s = nullptr;
-                if (alloc_ids(c, &specs[i].out_r, counts[i]) != hipSuccess ||
-                    alloc_ids(c, &specs[i].out_s, counts[i]) != hipSuccess) {
-                    return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
-                }
-                specs[i].cap = counts[i];
+                VJ_TRY(regrow(c, specs[i], counts[i]));
                 pl.joins[i].out_r = specs[i].out_r;
                 pl.joins[i].out_s = specs[i].out_s;
                 pl.joins[i].cap = specs[i].cap;

@@ -511,6 +511,13 @@ __global__ __launch_bounds__(256) void k_stage_copy(unsigned long long *dst, con
         dst[i] = src[i];
 }
 
+// Flat form: clears the table.
+__global__ __launch_bounds__(256) void k_flat_begin(FlatArgs a) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const gptr<u32x4> t = (gptr<u32x4>)a.slots;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.zero_words; i += gridDim.x * 256) t[i] = u32x4{0, 0, 0, 0};
+}
+
 // Resets the queue and the output counters to run build+probe again (after
 // an output buffer was found too small).
 __global__ void k_reset_probe(PipeArgs a) {
@@ -578,6 +585,19 @@ hipError_t launch_direct(const DirectArgs &d, const LaunchShape &sh, int blocks,
     case HP_FNV: return StageLaunch<HP_FNV>::direct(d, sh, blocks, s);
     case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::direct(d, sh, blocks, s);
     case HP_GENERIC: return StageLaunch<HP_GENERIC>::direct(d, sh, blocks, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s) {
+    const uint32_t blocks = (a.zero_words + 1023) / 1024;
+    hipLaunchKernelGGL(k_flat_begin, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, s, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    switch (sh.hp) {
+    case HP_FNV: return StageLaunch<HP_FNV>::flat(a, sh, s);
+    case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::flat(a, sh, s);
+    case HP_GENERIC: return StageLaunch<HP_GENERIC>::flat(a, sh, s);
     }
     return hipErrorInvalidValue;
 }

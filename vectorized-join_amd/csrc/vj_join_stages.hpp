@@ -1208,6 +1208,205 @@ __global__ __launch_bounds__(probe_threads(PV), (probe_waves_per_simd<HP, KW * N
     (void)finish_block(t.done, &a.ctl->done, a.out_count, a.down, a.down_words);
 }
 
+// ---------------------------------------------------------------------------
+// Flat form: one hash table in memory that an XCD's L2 holds
+// ---------------------------------------------------------------------------
+
+// Build sides of some thousand rows up to flat_max_rows: too many for an LDS
+// table, so few that partitioning costs more in launches and passes than it
+// saves. The table is open-addressed, at most half full: 8-byte slots {row + 1,
+// key} for 4-byte keys, in pairs read with one 16-byte load, 16-byte slots
+// {key, row + 1} for 8-byte keys, and {tag, row + 1} for wider ones, whose
+// matches are verified against the build columns. Equal keys are chained behind
+// the slot's row (nxt). Every probe row costs one random 16-byte read of the L2
+// (measured 150 G rows/s over a table of up to 2 MiB, 131 at 4 MiB, 92 at 8
+// MiB, 50 beyond), the probe side is read once and in order, and so are its
+// matches written.
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// What a slot holds of a key: the key itself up to 8 bytes, else a 64-bit mix of it.
+template <int KW, int NC> __device__ __forceinline__ uint64_t flat_word(const Key<KW, NC> &k) {
+    if constexpr (KW * NC == 4) return k.c[0];
+    else if constexpr (KW == 8 && NC == 1) return k.c[0];
+    else if constexpr (KW == 4 && NC == 2) return (uint64_t)k.c[0] | (uint64_t)k.c[1] << 32;
+    else {
+        uint64_t m = 0;
+#pragma unroll
+        for (int c = 0; c < NC; c++) m = (m ^ (uint64_t)k.c[c]) * 0x9E3779B97F4A7C15ull + (m >> 29);
+        return m;
+    }
+}
+
+template <int HP, int KW, int NC>
+__global__ __launch_bounds__(kFlatThreads) void k_flat_build(FlatArgs a) {
+    const uint32_t i = blockIdx.x * kFlatThreads + threadIdx.x;
+    if (i >= (uint32_t)a.r.n) return;
+    const Key<KW, NC> k = load_key<KW, NC>(a.r, i);
+    const uint32_t row = i + 1, lo = hash_key_lo<HP, KW, NC>(k, a.hash);
+    // An empty slot takes the row; the slot of an equal key takes it by an
+    // exchange (one atomic, however many rows of that key arrive) and the row
+    // links to the one it replaced. Only the probe kernel follows links.
+    uint32_t behind = 0;
+    if constexpr (KW * NC == 4) {
+        unsigned long long *slots = reinterpret_cast<unsigned long long *>(a.slots);
+        const unsigned long long mine = (unsigned long long)flat_word(k) << 32 | row;
+        uint32_t p = chain_of(lo, 0, a.hshift) * 2;  // slots of a pair fill in order
+        while (true) {
+            const unsigned long long got = atomicCAS(&slots[p], 0ull, mine);
+            if (got == 0) break;
+            if ((uint32_t)(got >> 32) == (uint32_t)(mine >> 32)) {
+                behind = (uint32_t)atomicExch(&slots[p], mine);
+                break;
+            }
+            p = (p + 1) & a.mask;
+        }
+    } else {
+        uint32_t p = chain_of(lo, 0, a.hshift);
+        while (true) {
+            uint32_t *slot = a.slots + (uint64_t)p * 4;  // {word lo, word hi, row, -}
+            const uint32_t got = atomicCAS(&slot[2], 0u, row);
+            if (got == 0) {
+                *reinterpret_cast<uint64_t *>(slot) = flat_word(k);  // the slot's key never changes again
+                break;
+            }
+            // the occupant's key, from the build side itself (the slot may not hold it yet)
+            if (key_eq<KW, NC>(k, load_key<KW, NC>(a.r, got - 1))) {
+                behind = atomicExch(&slot[2], row);
+                break;
+            }
+            p = (p + 1) & a.mask;
+        }
+    }
+    a.nxt[i] = behind;
+    if (behind) *a.dup = 1;
+}
+
+template <int HP, int KW, int NC, int U>
+__global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
+    constexpr int WAVES = kFlatThreads / 64;
+    constexpr bool K4 = KW * NC == 4, WIDE = KW * NC > 8;
+    __shared__ uint32_t wave_count[WAVES];
+    __shared__ unsigned long long out_base;
+    __shared__ uint32_t last;
+    const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const GKeys<KW, NC> sk = uniform_keys<KW, NC>(a.s), rk = uniform_keys<KW, NC>(a.r);
+    const gptr<const u32x4> slots = (gptr<const u32x4>)a.slots;
+    const gptr<const uint32_t> nxt = to_global(a.nxt);
+    const uint32_t n = (uint32_t)a.s.n, mask = a.mask, hshift = a.hshift;
+    const bool dup = *a.dup != 0;
+    // a wave's rows are consecutive, and so are its matches
+    const uint32_t row0 = blockIdx.x * (kFlatThreads * U) + w * 64 * U + lane;
+    Key<KW, NC> k[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) k[u] = load_key<KW, NC>(sk, row0 + u * 64 < n ? row0 + u * 64 : 0u);
+    uint32_t p[U], f[U];  // next slot (pair) to read, ~0: done; matched build row + 1
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t h = chain_of(hash_key_lo<HP, KW, NC>(k[u], a.hash), 0, hshift);
+        p[u] = row0 + u * 64 < n ? h : ~0u;
+        f[u] = 0;
+    }
+    while (true) {
+        bool any = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) any |= p[u] != ~0u;
+        if (!__ballot(any)) break;
+        u32x4 e[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) e[u] = slots[p[u] != ~0u ? p[u] : 0u];  // rows that are done: one shared line
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool live = p[u] != ~0u;
+            bool end;
+            uint32_t hit;
+            if constexpr (K4) {
+                const uint32_t key = (uint32_t)k[u].c[0];
+                hit = e[u].x && e[u].y == key ? e[u].x : (e[u].z && e[u].w == key ? e[u].z : 0u);
+                end = e[u].x == 0 || e[u].z == 0;
+            } else {
+                const uint64_t word = flat_word(k[u]);
+                hit = e[u].z && e[u].x == (uint32_t)word && e[u].y == (uint32_t)(word >> 32) ? e[u].z : 0u;
+                end = e[u].z == 0;
+                if constexpr (WIDE)
+                    if (live && hit && !key_eq<KW, NC>(k[u], load_key<KW, NC>(rk, hit - 1))) hit = 0;  // another key of the same mix
+            }
+            f[u] = live ? hit : f[u];
+            p[u] = !live || hit || end ? ~0u : (p[u] + 1) & (K4 ? mask >> 1 : mask);
+        }
+    }
+    uint32_t c = 0, cu[U];  // matches of the lane, of each of its rows
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        cu[u] = f[u] != 0;
+        if (dup) {  // uniform: rows of an equal key behind the match
+            uint32_t x = f[u];
+            while (x && cu[u] <= kFlatChain) {
+                x = nxt[x - 1];
+                cu[u] += x != 0;
+            }
+            // too many to follow one by one: the host runs the join in the pipeline (with the top bit of
+            // the count set no reservation is below any capacity, so nothing more is written)
+            if (x) atomicOr(a.count, kFlatGiveUp);
+        }
+        c += cu[u];
+    }
+    c = wave_sum<64>(c);
+    if (lane == 0) wave_count[w] = c;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t sum = 0;
+        for (int x = 0; x < WAVES; x++) sum += wave_count[x];
+        out_base = sum ? atomicAdd(a.count, (unsigned long long)sum) : 0;
+    }
+    const gptr<const uint32_t> rid = uniform_global(a.r.rowids), sid = uniform_global(a.s.rowids);
+    uint32_t r[U], s[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t i = row0 + u * 64;
+        s[u] = sid ? sid[i < n ? i : 0u] : i;
+        r[u] = rid ? rid[f[u] ? f[u] - 1 : 0u] : f[u] - 1;
+    }
+    __syncthreads();
+    if (c) {
+        WalkArgs wa;
+        wa.out_r = uniform_global(a.out_r);
+        wa.out_s = uniform_global(a.out_s);
+        wa.cap = uniform(a.cap);
+        const uint32_t ob1 = a.one_based;
+        Emitter em;
+        em.pos = out_base;
+        for (uint32_t x = 0; x < w; x++) em.pos += wave_count[x];
+        if (!dup) {  // uniform
+#pragma unroll
+            for (int u = 0; u < U; u++) em.put(f[u] != 0, r[u] + ob1, s[u] + ob1, wa);
+        } else {
+            // each lane writes its rows' matches by itself, behind those of the lanes below: no state
+            // of the wave is carried through a loop that lanes leave at different times
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t inc = wave_incl_scan(cu[u]);
+                unsigned long long o = em.pos + inc - cu[u];
+                uint32_t x = f[u], id = r[u];
+                for (uint32_t m = 0; m < cu[u]; m++) {
+                    if (o < wa.cap) {
+                        wa.out_r[o] = id + ob1;
+                        wa.out_s[o] = s[u] + ob1;
+                    }
+                    o++;
+                    x = nxt[x - 1];
+                    if (x) id = rid ? rid[x - 1] : x - 1;
+                }
+                em.pos += __shfl(inc, 63, 64);
+            }
+        }
+    }
+    if (finish_block(last, a.done, a.count, a.down, 1)) {
+        __syncthreads();
+        if (tid == 0) *a.count = 0;  // for the next join
+    }
+}
+
 // Dispatch over the key shape (key width, key columns).
 template <typename F> hipError_t dispatch_keys(const LaunchShape &sh, F &&f) {
 #define VJ_CASE(KW, NC) \
@@ -1311,6 +1510,22 @@ template <int HP> hipError_t StageLaunch<HP>::direct(const DirectArgs &d, const 
             hipLaunchKernelGGL((k_direct<HP, KW, NC, 1>), dim3(blocks), dim3(probe_threads(1)), lds, s, d);
         else
             hipLaunchKernelGGL((k_direct<HP, KW, NC, 0>), dim3(blocks), dim3(probe_threads(0)), lds, s, d);
+        return hipGetLastError();
+    });
+}
+
+template <int HP> hipError_t StageLaunch<HP>::flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s) {
+    return dispatch_keys(sh, [&]<int KW, int NC>() {
+        constexpr int U = KW * NC <= 8 ? 8 : 4;
+        const uint32_t n = (uint32_t)a.s.n;
+        hipLaunchKernelGGL((k_flat_build<HP, KW, NC>), dim3(((uint32_t)a.r.n + kFlatThreads - 1) / kFlatThreads), dim3(kFlatThreads), 0, s, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        // few probe rows: fewer per thread, so that more CUs take part
+        if (n <= 1u << 20)
+            hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, 2>), dim3((n - 1) / (kFlatThreads * 2) + 1), dim3(kFlatThreads), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, U>), dim3((n - 1) / (kFlatThreads * U) + 1), dim3(kFlatThreads), 0, s, a);
         return hipGetLastError();
     });
 }

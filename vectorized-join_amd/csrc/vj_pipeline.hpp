@@ -256,6 +256,35 @@ struct DirectArgs {
     HashCfg hash;
 };
 
+// The flat form (k_flat_build, k_flat_probe): slots of the table in 16-byte
+// groups, zero before the build; links of equal keys, one per build row.
+constexpr int kFlatThreads = 512;
+constexpr uint32_t kFlatChain = 64;                     // rows of one key followed link by link
+constexpr unsigned long long kFlatGiveUp = 1ull << 63;  // in the count: a chain was longer
+constexpr uint64_t kFlatTableBytes = 4ull << 20;  // an XCD's L2
+__host__ __device__ constexpr int flat_slot_bytes(int key_bytes) { return key_bytes <= 4 ? 8 : 16; }
+// Build rows of the largest table: half full in pairs of 8-byte slots, a
+// quarter in single 16-byte ones, whose chains grow sooner (device us, flat and
+// pipeline: 2^18 x 2^24 4-byte keys 147 / 166; 2^16 x 2^20 8-byte keys 46 / 61,
+// 4 x u32 50 / 81; 2^17 x 2^20 8-byte keys, half full, 96 / 62).
+__host__ __device__ constexpr uint64_t flat_max_rows(int key_bytes) {
+    return kFlatTableBytes / flat_slot_bytes(key_bytes) / (key_bytes <= 4 ? 2 : 4);
+}
+struct FlatArgs {
+    TView r, s;
+    uint32_t *slots;
+    uint32_t *nxt;
+    uint32_t *dup;      // set when two build rows have equal keys
+    uint32_t mask;      // slots - 1
+    uint32_t hshift;    // 32 - log2 of the slots (of the pairs for 4-byte keys)
+    uint32_t *out_r, *out_s;
+    uint64_t cap;
+    uint32_t one_based;
+    uint32_t zero_words;  // 16-byte words from `slots` on to clear before the build (the table, then dup)
+    unsigned long long *count, *done, *down;  // as DirectArgs
+    HashCfg hash;
+};
+
 // Kernel launchers (vj_join_kernels.hip); all asynchronous on `s`.
 struct LaunchShape {
     int hp, kw, nc;  // hash path, key width, key columns
@@ -274,6 +303,7 @@ template <int HP> struct StageLaunch {
     static hipError_t fan(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
     static hipError_t probe(const PipeArgs &a, const LaunchShape &sh, int blocks, hipStream_t s);
     static hipError_t direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s);
+    static hipError_t flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s);
     static int probe_blocks_per_cu(const LaunchShape &sh);
 };
 extern template struct StageLaunch<HP_FNV>;
@@ -281,6 +311,7 @@ extern template struct StageLaunch<HP_XOR_HW>;
 extern template struct StageLaunch<HP_GENERIC>;
 hipError_t launch_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_scan(const PipeArgs &a, hipStream_t s);
+hipError_t launch_flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s);
 hipError_t launch_fan_begin(const PipeArgs &a, hipStream_t s);
 hipError_t launch_fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
