@@ -1288,8 +1288,10 @@ __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
     constexpr bool K4 = KW * NC == 4, WIDE = KW * NC > 8;
     __shared__ uint32_t wave_count[WAVES];
     __shared__ unsigned long long out_base;
-    __shared__ uint32_t last;
+    __shared__ uint32_t last, long_chain;
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    if (tid == 0) long_chain = 0;
+    __syncthreads();
     const GKeys<KW, NC> sk = uniform_keys<KW, NC>(a.s), rk = uniform_keys<KW, NC>(a.r);
     const gptr<const u32x4> slots = (gptr<const u32x4>)a.slots;
     const gptr<const uint32_t> nxt = to_global(a.nxt);
@@ -1345,9 +1347,7 @@ __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
                 x = nxt[x - 1];
                 cu[u] += x != 0;
             }
-            // too many to follow one by one: the host runs the join in the pipeline (with the top bit of
-            // the count set no reservation is below any capacity, so nothing more is written)
-            if (x) atomicOr(a.count, kFlatGiveUp);
+            if (x) long_chain = 1;
         }
         c += cu[u];
     }
@@ -1357,7 +1357,11 @@ __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
     if (tid == 0) {
         uint32_t sum = 0;
         for (int x = 0; x < WAVES; x++) sum += wave_count[x];
-        out_base = sum ? atomicAdd(a.count, (unsigned long long)sum) : 0;
+        // A key with too many rows to follow one by one: the host runs the join in the pipeline (with the top
+        // bit of the count set no reservation is below any capacity, so nothing more is written). Both atomics
+        // are waited for here: this thread counts the block as ended after them.
+        if (long_chain) out_base = atomicOr(a.count, kFlatGiveUp) | kFlatGiveUp;
+        else out_base = sum ? atomicAdd(a.count, (unsigned long long)sum) : 0;
     }
     const gptr<const uint32_t> rid = uniform_global(a.r.rowids), sid = uniform_global(a.s.rowids);
     uint32_t r[U], s[U];
