@@ -1147,24 +1147,70 @@ bool may_run_direct(const vj_ctx *c, const Plan &pl) {
     return !r.b1 && !s.b1 && r.n > 0 && s.n > 0 && r.n <= pl.joins[0].cap_r;
 }
 
-// Whether a join runs in the flat form: a single planner-driven join (no
-// plan of the caller's or the tuner's) whose build side is past an LDS table
-// and whose table an XCD's L2 holds. Under a budget and with per-stage timing
-// the pipeline runs as ever.
-bool may_run_flat(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_opts *o) {
-    if (c->budget || c->profiling || !c->direct || !c->na_stage || specs.size() != 1 || specs[0].res || specs[0].keep) return false;
-    if (o->passes != -1 || o->bits1 || o->bits2 || o->tile || o->table || o->layout == VJ_LAYOUT_REGIONS) return false;
-    const vj_table *r = specs[0].r, *s = specs[0].s;
-    const int kb = s->key_width * s->n_cols;
-    if (r->n_rows <= (uint64_t)build_cap(kb) * 3 / 4 || r->n_rows > flat_max_rows(kb) || s->n_rows == 0) return false;
-    HashCfg h;
-    if (make_hash_cfg(&o->hash, s, &h).failed()) return false;
-    const uint64_t key = tune_key(r->n_rows, kb, hash_path(h));
+// Whether this context's planner-driven joins may run in the flat form: no plan
+// of the caller's, no budget and no per-stage timing (there the pipeline runs as
+// ever).
+bool flat_allowed(const vj_ctx *c, const vj_join_opts *o) {
+    if (c->budget || c->profiling || !c->direct || !c->na_stage) return false;
+    return o->passes == -1 && !o->bits1 && !o->bits2 && !o->tile && !o->table && o->layout != VJ_LAYOUT_REGIONS;
+}
+
+// Whether the size class of a build side stays in the flat form: no tuned plan,
+// no long chains lately.
+bool flat_class_ok(vj_ctx *c, uint64_t key) {
     if (c->tuned.count(key)) return false;
     auto it = c->flat_skip.find(key);
     if (it == c->flat_skip.end()) return true;
     if (--it->second <= 0) c->flat_skip.erase(it);
     return false;
+}
+
+// Whether a join runs in the flat form: a single join whose build side is
+// past an LDS table and whose table an XCD's L2 holds.
+bool may_run_flat(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_opts *o) {
+    if (!flat_allowed(c, o) || specs.size() != 1 || specs[0].res || specs[0].keep) return false;
+    const vj_table *r = specs[0].r, *s = specs[0].s;
+    const int kb = s->key_width * s->n_cols;
+    if (r->n_rows <= (uint64_t)build_cap(kb) * 3 / 4 || r->n_rows > flat_max_rows(kb) || s->n_rows == 0) return false;
+    HashCfg h;
+    if (make_hash_cfg(&o->hash, s, &h).failed()) return false;
+    return flat_class_ok(c, tune_key(r->n_rows, kb, hash_path(h)));
+}
+
+// Slots of the table of n build rows: a quarter full where that still fits, else
+// up to half; in a batch single slots are a quarter full, and pairs half, as more
+// tables share an L2. At least two pairs: the kernels shift a 32-bit product by 32
+// less their log2.
+uint64_t flat_slots(uint64_t n, int kb, bool batch) {
+    const uint64_t slots = std::max<uint64_t>(4, 1ull << ceil_log2(2 * n));
+    return batch && kb <= 4 ? slots : slots * 2 * flat_slot_bytes(kb) <= kFlatTableBytes ? slots * 2 : slots;
+}
+
+// The kernels' arguments of one join but for its memory.
+FlatArgs flat_args(const JoinSpec &js, const vj_join_opts *o, const HashCfg &h, bool batch) {
+    FlatArgs a;
+    memset(&a, 0, sizeof(a));
+    a.hash = h;
+    a.r = to_view(js.r);
+    a.s = to_view(js.s);
+    const int kb = js.s->key_width * js.s->n_cols;
+    const uint64_t slots = flat_slots(a.r.n, kb, batch);
+    a.mask = (uint32_t)(slots - 1);
+    a.hshift = 32u - (uint32_t)ceil_log2(kb <= 4 ? slots / 2 : slots);
+    a.one_based = o->one_based ? 1 : 0;
+    a.out_r = js.out_r;
+    a.out_s = js.out_s;
+    a.cap = js.cap;
+    return a;
+}
+
+LaunchShape flat_shape(const vj_ctx *c, const vj_table *t, const HashCfg &h) {
+    LaunchShape sh{};
+    sh.hp = hash_path(h);
+    sh.kw = t->key_width;
+    sh.nc = t->n_cols;
+    sh.cus = c->cus;
+    return sh;
 }
 
 // *ran: false if the build side has more equal keys than the form follows; the
@@ -1173,30 +1219,18 @@ Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std:
              int *retries_out, bool *ran) {
     *ran = true;
     VJ_TRY(check_pair(js.r, js.s));
-    FlatArgs a;
-    memset(&a, 0, sizeof(a));
-    VJ_TRY(make_hash_cfg(&o->hash, js.s, &a.hash));
-    a.r = to_view(js.r);
-    a.s = to_view(js.s);
-    LaunchShape sh{};
-    sh.hp = hash_path(a.hash);
-    sh.kw = js.s->key_width;
-    sh.nc = js.s->n_cols;
-    sh.cus = c->cus;
+    HashCfg h;
+    VJ_TRY(make_hash_cfg(&o->hash, js.s, &h));
+    FlatArgs a = flat_args(js, o, h, false);
+    const LaunchShape sh = flat_shape(c, js.s, h);
     const int kb = sh.kw * sh.nc;
-    // a quarter full where that still fits, else up to half
-    uint64_t slots = 1ull << ceil_log2(2 * a.r.n);
-    if (slots * 2 * flat_slot_bytes(kb) <= kFlatTableBytes) slots *= 2;
-    const size_t table = slots * flat_slot_bytes(kb), links = align_up(a.r.n * 4);
+    const size_t table = ((size_t)a.mask + 1) * flat_slot_bytes(kb), links = align_up(a.r.n * 4);
     VJ_TRY(ensure(c->tuples, table + kAlign + links, true));
     char *m = static_cast<char *>(c->tuples.p);
     a.slots = reinterpret_cast<uint32_t *>(m);
     a.dup = reinterpret_cast<uint32_t *>(m + table);
     a.nxt = reinterpret_cast<uint32_t *>(m + table + kAlign);
-    a.mask = (uint32_t)(slots - 1);
-    a.hshift = 32u - (uint32_t)ceil_log2(kb <= 4 ? slots / 2 : slots);
     a.zero_words = (uint32_t)((table + 16) / 16);
-    a.one_based = o->one_based ? 1 : 0;
     a.count = static_cast<unsigned long long *>(c->direct);
     a.done = a.count + 32;
     a.down = static_cast<unsigned long long *>(c->na_stage);
@@ -1238,6 +1272,92 @@ Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std:
     sm.bytes_total = sm.bytes_build_probe;
     sm.gbps_total = gbps(sm.bytes_total, sm.ms_total);
     sm.probe_tuples_per_s = sm.ms_total > 0 ? (double)sm.probe_rows / (sm.ms_total * 1e-3) : 0.0;
+    return Err::ok();
+}
+
+// Whether a batch runs in the flat form as a whole: every join's table would
+// fit an XCD's L2, and all of them together about fit the L2s of the chip.
+bool may_run_flat_batch(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_opts *o, HashCfg *h) {
+    if (!flat_allowed(c, o) || specs.size() < 2) return false;
+    const vj_table *t0 = specs[0].s;
+    if (check_table(t0).failed() || make_hash_cfg(&o->hash, t0, h).failed()) return false;
+    const int kb = t0->key_width * t0->n_cols;
+    uint64_t bytes = 0, blocks = 0;
+    for (const JoinSpec &js : specs) {
+        if (js.res || js.keep || check_pair(js.r, js.s).failed()) return false;
+        if (js.s->n_cols != t0->n_cols || js.s->key_width != t0->key_width || (js.s->key_signed != 0) != (t0->key_signed != 0)) return false;
+        if (js.r->n_rows > flat_max_rows(kb)) return false;
+        bytes += flat_slots(js.r->n_rows, kb, true) * flat_slot_bytes(kb);
+        blocks += js.r->n_rows && js.s->n_rows ? js.s->n_rows / (kFlatThreads * flat_batch_rows(kb)) + 1 : 0;
+    }
+    if (!blocks || blocks >> 31 || bytes > flat_batch_bytes(kb)) return false;
+    return flat_class_ok(c, tune_key(largest_build(specs), kb, hash_path(*h)));
+}
+
+// *ran: as run_flat, over all joins.
+Err run_flat_batch(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_opts *o, const HashCfg &h, hipStream_t s,
+                   std::vector<uint64_t> &counts, bool *ran) {
+    *ran = true;
+    const LaunchShape sh = flat_shape(c, specs[0].s, h);
+    const int kb = sh.kw * sh.nc;
+    const size_t n = specs.size();
+    // tables, then a dup word each (these are cleared), then the links
+    std::vector<FlatArgs> args(n);
+    std::vector<uint32_t> build0(n + 1, 0), probe0(n + 1, 0);
+    std::vector<size_t> at(n), links_at(n);
+    size_t tables = 0, links = 0;
+    for (size_t i = 0; i < n; i++) {
+        args[i] = flat_args(specs[i], o, h, true);
+        const uint64_t nr = args[i].r.n, ns = args[i].s.n;
+        at[i] = tables;
+        tables += ((size_t)args[i].mask + 1) * flat_slot_bytes(kb);
+        links_at[i] = links;
+        links += align_up(nr * 4);
+        const uint64_t per = (uint64_t)kFlatThreads * flat_batch_rows(kb);
+        build0[i + 1] = build0[i] + (uint32_t)(ns ? (nr + kFlatThreads - 1) / kFlatThreads : 0);
+        probe0[i + 1] = probe0[i] + (uint32_t)(nr ? (ns + per - 1) / per : 0);
+    }
+    const size_t dups = align_up(n * 4);
+    VJ_TRY(ensure(c->tuples, tables + dups + links, true));
+    const size_t o_b0 = align_up(n * sizeof(FlatArgs)), o_p0 = align_up(o_b0 + (n + 1) * 4), up = align_up(o_p0 + (n + 1) * 4);
+    const size_t o_counts = up, o_done = align_up(o_counts + n * 8), meta = o_done + kAlign;
+    VJ_TRY(ensure(c->meta, meta, true));
+    VJ_TRY(ensure_pinned(c, meta));
+    char *m = static_cast<char *>(c->tuples.p), *d = static_cast<char *>(c->meta.p), *p = static_cast<char *>(c->pinned);
+    FlatBatch b;
+    memset(&b, 0, sizeof(b));
+    b.joins = reinterpret_cast<const FlatArgs *>(d);
+    b.build0 = reinterpret_cast<const uint32_t *>(d + o_b0);
+    b.probe0 = reinterpret_cast<const uint32_t *>(d + o_p0);
+    b.n_joins = (uint32_t)n;
+    b.build_blocks = build0[n];
+    b.probe_blocks = probe0[n];
+    b.up_words = (uint32_t)(up / 8);
+    b.up_dst = reinterpret_cast<unsigned long long *>(d);
+    b.up_src = reinterpret_cast<const unsigned long long *>(p);
+    b.zero = reinterpret_cast<uint32_t *>(m);
+    b.zero_words = (tables + dups) / 16;
+    b.counts = reinterpret_cast<unsigned long long *>(d + o_counts);
+    b.done = reinterpret_cast<unsigned long long *>(d + o_done);
+    b.down = reinterpret_cast<unsigned long long *>(p + o_counts);
+    for (size_t i = 0; i < n; i++) {
+        args[i].slots = reinterpret_cast<uint32_t *>(m + at[i]);
+        args[i].dup = reinterpret_cast<uint32_t *>(m + tables) + i;
+        args[i].nxt = reinterpret_cast<uint32_t *>(m + tables + dups + links_at[i]);
+        args[i].count = b.counts + i;
+    }
+    memcpy(p, args.data(), n * sizeof(FlatArgs));
+    memcpy(p + o_b0, build0.data(), (n + 1) * 4);
+    memcpy(p + o_p0, probe0.data(), (n + 1) * 4);
+    VJ_LAUNCH(launch_flat_batch(b, sh, s));
+    VJ_HIP_TRY(hipStreamSynchronize(s));
+    counts.assign(b.down, b.down + n);
+    for (uint64_t x : counts) {
+        if (x & kFlatGiveUp) {
+            c->flat_skip[tune_key(largest_build(specs), kb, sh.hp)] = 64;
+            *ran = false;
+        }
+    }
     return Err::ok();
 }
 
@@ -1287,6 +1407,12 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
     if (may_run_flat(c, specs, o)) {
         bool ran = false;
         VJ_TRY(run_flat(c, specs[0], o, s, counts, grow, retries_out, &ran));
+        if (ran) return Err::ok();
+    }
+    HashCfg fh;
+    if (gmode == GRAPH_OFF && !grow && may_run_flat_batch(c, specs, o, &fh)) {
+        bool ran = false;
+        VJ_TRY(run_flat_batch(c, specs, o, fh, s, counts, &ran));
         if (ran) return Err::ok();
     }
     Plan pl;

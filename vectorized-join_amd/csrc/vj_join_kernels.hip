@@ -518,6 +518,17 @@ __global__ __launch_bounds__(256) void k_flat_begin(FlatArgs a) {
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.zero_words; i += gridDim.x * 256) t[i] = u32x4{0, 0, 0, 0};
 }
 
+// A batch: also fetches its arguments and clears the counts.
+__global__ __launch_bounds__(256) void k_flat_begin_batch(FlatBatch b) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const uint32_t i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+    for (uint32_t i = i0; i < b.up_words; i += step) b.up_dst[i] = b.up_src[i];
+    for (uint32_t j = i0; j < b.n_joins; j += step) b.counts[j] = 0;
+    if (i0 == 0) *b.done = 0;
+    const gptr<u32x4> t = (gptr<u32x4>)b.zero;
+    for (uint64_t i = i0; i < b.zero_words; i += step) t[i] = u32x4{0, 0, 0, 0};
+}
+
 // Resets the queue and the output counters to run build+probe again (after
 // an output buffer was found too small).
 __global__ void k_reset_probe(PipeArgs a) {
@@ -598,6 +609,19 @@ hipError_t launch_flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s) 
     case HP_FNV: return StageLaunch<HP_FNV>::flat(a, sh, s);
     case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::flat(a, sh, s);
     case HP_GENERIC: return StageLaunch<HP_GENERIC>::flat(a, sh, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_flat_batch(const FlatBatch &b, const LaunchShape &sh, hipStream_t s) {
+    const uint64_t blocks = (b.zero_words + 1023) / 1024;
+    hipLaunchKernelGGL(k_flat_begin_batch, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s, b);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    switch (sh.hp) {
+    case HP_FNV: return StageLaunch<HP_FNV>::flat_batch(b, sh, s);
+    case HP_XOR_HW: return StageLaunch<HP_XOR_HW>::flat_batch(b, sh, s);
+    case HP_GENERIC: return StageLaunch<HP_GENERIC>::flat_batch(b, sh, s);
     }
     return hipErrorInvalidValue;
 }

@@ -1238,9 +1238,8 @@ template <int KW, int NC> __device__ __forceinline__ uint64_t flat_word(const Ke
     }
 }
 
-template <int HP, int KW, int NC>
-__global__ __launch_bounds__(kFlatThreads) void k_flat_build(FlatArgs a) {
-    const uint32_t i = blockIdx.x * kFlatThreads + threadIdx.x;
+template <int HP, int KW, int NC> __device__ __forceinline__ void flat_build_block(const FlatArgs &a, uint32_t block) {
+    const uint32_t i = block * kFlatThreads + threadIdx.x;
     if (i >= (uint32_t)a.r.n) return;
     const Key<KW, NC> k = load_key<KW, NC>(a.r, i);
     const uint32_t row = i + 1, lo = hash_key_lo<HP, KW, NC>(k, a.hash);
@@ -1282,13 +1281,16 @@ __global__ __launch_bounds__(kFlatThreads) void k_flat_build(FlatArgs a) {
     if (behind) *a.dup = 1;
 }
 
-template <int HP, int KW, int NC, int U>
-__global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
+template <int HP, int KW, int NC> __global__ __launch_bounds__(kFlatThreads) void k_flat_build(FlatArgs a) {
+    flat_build_block<HP, KW, NC>(a, blockIdx.x);
+}
+
+template <int HP, int KW, int NC, int U> __device__ __forceinline__ void flat_probe_block(const FlatArgs &a, uint32_t block) {
     constexpr int WAVES = kFlatThreads / 64;
     constexpr bool K4 = KW * NC == 4, WIDE = KW * NC > 8;
     __shared__ uint32_t wave_count[WAVES];
     __shared__ unsigned long long out_base;
-    __shared__ uint32_t last, long_chain;
+    __shared__ uint32_t long_chain;
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     if (tid == 0) long_chain = 0;
     __syncthreads();
@@ -1298,7 +1300,7 @@ __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
     const uint32_t n = (uint32_t)a.s.n, mask = a.mask, hshift = a.hshift;
     const bool dup = *a.dup != 0;
     // a wave's rows are consecutive, and so are its matches
-    const uint32_t row0 = blockIdx.x * (kFlatThreads * U) + w * 64 * U + lane;
+    const uint32_t row0 = block * (kFlatThreads * U) + w * 64 * U + lane;
     Key<KW, NC> k[U];
 #pragma unroll
     for (int u = 0; u < U; u++) k[u] = load_key<KW, NC>(sk, row0 + u * 64 < n ? row0 + u * 64 : 0u);
@@ -1405,10 +1407,40 @@ __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
             }
         }
     }
+}
+
+template <int HP, int KW, int NC, int U> __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
+    __shared__ uint32_t last;
+    flat_probe_block<HP, KW, NC, U>(a, blockIdx.x);
     if (finish_block(last, a.done, a.count, a.down, 1)) {
         __syncthreads();
-        if (tid == 0) *a.count = 0;  // for the next join
+        if (threadIdx.x == 0) *a.count = 0;  // for the next join
     }
+}
+
+// A batch's blocks stand join after join in one line, of which each XCD takes
+// one eighth from its start on: the few joins an XCD works on at a time have
+// their tables in its L2 and in no other (a grid is a multiple of kXcds).
+// The join and the block in it; false: past the line's end.
+__device__ __forceinline__ bool flat_batch_at(const uint32_t *first, uint32_t n_joins, uint32_t total, uint32_t &j, uint32_t &block) {
+    const uint32_t at = blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+    if (at >= total) return false;
+    j = uniform(wave_upper_index(first, n_joins, at));
+    block = at - first[j];
+    return true;
+}
+
+template <int HP, int KW, int NC> __global__ __launch_bounds__(kFlatThreads) void k_flat_build_batch(FlatBatch b) {
+    uint32_t j, block;
+    if (flat_batch_at(b.build0, b.n_joins, b.build_blocks, j, block)) flat_build_block<HP, KW, NC>(b.joins[j], block);
+}
+
+template <int HP, int KW, int NC> __global__ __launch_bounds__(kFlatThreads) void k_flat_probe_batch(FlatBatch b) {
+    __shared__ uint32_t last;
+    uint32_t j, block;
+    if (flat_batch_at(b.probe0, b.n_joins, b.probe_blocks, j, block))
+        flat_probe_block<HP, KW, NC, flat_batch_rows(KW * NC)>(b.joins[j], block);
+    (void)finish_block(last, b.done, b.counts, b.down, b.n_joins);
 }
 
 // Dispatch over the key shape (key width, key columns).
@@ -1530,6 +1562,17 @@ template <int HP> hipError_t StageLaunch<HP>::flat(const FlatArgs &a, const Laun
             hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, 2>), dim3((n - 1) / (kFlatThreads * 2) + 1), dim3(kFlatThreads), 0, s, a);
         else
             hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, U>), dim3((n - 1) / (kFlatThreads * U) + 1), dim3(kFlatThreads), 0, s, a);
+        return hipGetLastError();
+    });
+}
+
+template <int HP> hipError_t StageLaunch<HP>::flat_batch(const FlatBatch &b, const LaunchShape &sh, hipStream_t s) {
+    auto grid = [](uint32_t blocks) { return dim3((blocks + kXcds - 1) / kXcds * kXcds); };
+    return dispatch_keys(sh, [&]<int KW, int NC>() {
+        hipLaunchKernelGGL((k_flat_build_batch<HP, KW, NC>), grid(b.build_blocks), dim3(kFlatThreads), 0, s, b);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((k_flat_probe_batch<HP, KW, NC>), grid(b.probe_blocks), dim3(kFlatThreads), 0, s, b);
         return hipGetLastError();
     });
 }

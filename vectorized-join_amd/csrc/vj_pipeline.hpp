@@ -262,6 +262,15 @@ constexpr int kFlatThreads = 512;
 constexpr uint32_t kFlatChain = 64;                     // rows of one key followed link by link
 constexpr unsigned long long kFlatGiveUp = 1ull << 63;  // in the count: a chain was longer
 constexpr uint64_t kFlatTableBytes = 4ull << 20;  // an XCD's L2
+// All tables of a batch, beyond which the pipeline is the faster one (us a call,
+// flat and pipeline, build sides log-uniform from 2^10, probe sides 4-16 times
+// as large): 4-byte keys, 64 joins of up to 2^14 rows (8 MB) 105 / 150, of 2^16
+// (21 MB) 186 / 219, of 2^18 (63 MB) 434 / 361, 16 of 2^18 (14 MB) 131 / 141;
+// 8-byte keys, 20 joins of up to 2^15 rows (13 MB) 72 / 101, 16 of 2^16 (23 MB)
+// 122 / 113, 64 of 2^16 (85 MB) 304 / 227; 4 x u32, 40 of 2^14 (18 MB)
+// 118 / 158, of 2^16 (57 MB) 206 / 198; 2 x u64, 30 of 2^15 (24 MB) 124 / 159;
+// two joins of 2048 rows 34 / 69.
+__host__ __device__ constexpr uint64_t flat_batch_bytes(int key_bytes) { return (key_bytes > 4 && key_bytes <= 8 ? 16ull : 32ull) << 20; }
 __host__ __device__ constexpr int flat_slot_bytes(int key_bytes) { return key_bytes <= 4 ? 8 : 16; }
 // Build rows of the largest table: half full in pairs of 8-byte slots, a
 // quarter in single 16-byte ones, whose chains grow sooner (device us, flat and
@@ -270,6 +279,8 @@ __host__ __device__ constexpr int flat_slot_bytes(int key_bytes) { return key_by
 __host__ __device__ constexpr uint64_t flat_max_rows(int key_bytes) {
     return kFlatTableBytes / flat_slot_bytes(key_bytes) / (key_bytes <= 4 ? 2 : 4);
 }
+// Probe rows per thread of a batch's joins.
+__host__ __device__ constexpr int flat_batch_rows(int key_bytes) { return key_bytes <= 8 ? 8 : 4; }
 struct FlatArgs {
     TView r, s;
     uint32_t *slots;
@@ -283,6 +294,20 @@ struct FlatArgs {
     uint32_t zero_words;  // 16-byte words from `slots` on to clear before the build (the table, then dup)
     unsigned long long *count, *done, *down;  // as DirectArgs
     HashCfg hash;
+};
+
+// A batch in the flat form: its joins' arguments in memory, a grid over all of
+// their build blocks and one over their probe blocks.
+struct FlatBatch {
+    const FlatArgs *joins;
+    const uint32_t *build0, *probe0;  // [n_joins + 1] prefixes of the joins' blocks
+    uint32_t n_joins, build_blocks, probe_blocks;
+    uint32_t up_words;                // the arguments' and prefixes' way from the host's buffer, in 8-byte words
+    unsigned long long *up_dst;
+    const unsigned long long *up_src;
+    uint32_t *zero;                   // the tables and their dup words
+    uint64_t zero_words;              // in 16-byte words
+    unsigned long long *counts, *done, *down;
 };
 
 // Kernel launchers (vj_join_kernels.hip); all asynchronous on `s`.
@@ -304,6 +329,7 @@ template <int HP> struct StageLaunch {
     static hipError_t probe(const PipeArgs &a, const LaunchShape &sh, int blocks, hipStream_t s);
     static hipError_t direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s);
     static hipError_t flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s);
+    static hipError_t flat_batch(const FlatBatch &b, const LaunchShape &sh, hipStream_t s);
     static int probe_blocks_per_cu(const LaunchShape &sh);
 };
 extern template struct StageLaunch<HP_FNV>;
@@ -312,6 +338,7 @@ extern template struct StageLaunch<HP_GENERIC>;
 hipError_t launch_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_scan(const PipeArgs &a, hipStream_t s);
 hipError_t launch_flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s);
+hipError_t launch_flat_batch(const FlatBatch &b, const LaunchShape &sh, hipStream_t s);
 hipError_t launch_direct(const DirectArgs &d, const LaunchShape &sh, int blocks, hipStream_t s);
 hipError_t launch_fan_begin(const PipeArgs &a, hipStream_t s);
 hipError_t launch_fan_hist(const PipeArgs &a, const LaunchShape &sh, hipStream_t s);
