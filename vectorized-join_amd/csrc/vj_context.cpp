@@ -43,6 +43,8 @@ struct vj_ctx {
     int cus = 256;
     uint64_t budget = 0;
     bool profiling = false;
+    bool by_events = false;  // joins are timed by events in every form (vj_tune: forms are compared)
+    int clock_khz = 0;       // rate of the device clock (0: unknown)
     std::string last_error;
     vj_join_summary summary{};
     DevBuf tuples, counts, base, ptask, meta;
@@ -170,9 +172,6 @@ struct Plan {
     // meta layout
     size_t off_jobs = 0, off_joins = 0, off_cs = 0, off_hb0 = 0, off_pt0 = 0, off_pc0 = 0, upload_bytes = 0;
     size_t off_jtasks = 0, off_task0 = 0, off_count = 0, off_ctl = 0, meta_bytes = 0;
-    // Bytes downloaded after a launch: the match counts and the control words
-    // behind them (the queue's task total).
-    size_t down_bytes() const { return off_ctl + sizeof(Ctl) - off_count; }
 };
 
 int ceil_log2(uint64_t v) {
@@ -890,7 +889,7 @@ PipeArgs make_args(const Arenas &ar, const Plan &pl) {
     a.pass_tile = pass_tile(pl.kb, pl.shape.tile);
     a.regions = pl.regions ? 1u : 0u;
     a.down = reinterpret_cast<unsigned long long *>(ar.pinned + pl.off_count);
-    a.down_words = (uint32_t)(pl.down_bytes() / 8);
+    a.down_words = (uint32_t)((pl.off_ctl + offsetof(Ctl, t1) - pl.off_count) / 8);
     if (pl.fan) {
         a.up_dst = reinterpret_cast<unsigned long long *>(m);
         a.up_src = reinterpret_cast<const unsigned long long *>(ar.pinned);
@@ -942,11 +941,20 @@ int probe_grid(const vj_ctx *c, const Plan &pl) {
     return (int)std::max<uint64_t>(1, std::min(tasks, fit));
 }
 
+// Whether a pipeline's time comes from the clock its first and last kernels
+// read, not from events around it.
+bool timed_by_clock(const vj_ctx *c, const Plan &pl) { return pl.fan && !c->profiling && !c->by_events && c->clock_khz > 0; }
+
+double clock_ms(const vj_ctx *c, unsigned long long t0, unsigned long long t1) {
+    return c->clock_khz > 0 && t1 > t0 ? (double)(t1 - t0) / c->clock_khz : 0.0;
+}
+
 // Launches every stage on `s` (no host synchronisation). `events`: record
-// the start / end events (and the per-stage ones when profiling); off while
-// a graph is being captured.
+// the start / end events where they are read (and the per-stage ones when
+// profiling); off while a graph is being captured.
 Err launch_stages(vj_ctx *c, const Plan &pl, const PipeArgs &a, hipStream_t s, bool with_probe, bool events = true) {
     const bool prof = c->profiling && events;
+    if (timed_by_clock(c, pl)) events = false;
     if (events) VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
     if (pl.regions) {
         // region layout: counters zeroed, both passes reserve runs, then the task prefix
@@ -1074,8 +1082,9 @@ void stage_bytes(const Plan &pl, uint64_t matches, vj_join_summary &s) {
 
 double gbps(uint64_t bytes, double ms) { return ms > 0 ? (double)bytes / (ms * 1e-3) / 1e9 : 0.0; }
 
+// t0, t1: the device clock of a join that is timed by it.
 void fill_summary(vj_ctx *c, const Plan &pl, const JoinSpec &js, uint64_t matches, uint64_t tasks, int retries,
-                  bool replay, uint64_t scratch_bytes) {
+                  bool replay, uint64_t scratch_bytes, unsigned long long t0, unsigned long long t1) {
     vj_join_summary &s = c->summary;
     memset(&s, 0, sizeof(s));
     s.build_rows = js.res ? js.res->n : js.r->n_rows;
@@ -1088,7 +1097,7 @@ void fill_summary(vj_ctx *c, const Plan &pl, const JoinSpec &js, uint64_t matche
     s.retries = retries;
     s.partitions = pl.joins[0].nparts;
     s.tasks = tasks;
-    s.ms_total = elapsed(c->ev[EV_START], c->ev[EV_PROBE]);
+    s.ms_total = timed_by_clock(c, pl) ? clock_ms(c, t0, t1) : elapsed(c->ev[EV_START], c->ev[EV_PROBE]);
     if (c->profiling) {
         s.ms_histogram = elapsed(c->ev[EV_START], c->ev[EV_HIST]);
         s.ms_pass1 = elapsed(c->ev[EV_SCAN], c->ev[EV_P1]);
@@ -1142,7 +1151,7 @@ Err regrow(const vj_ctx *c, JoinSpec &js, uint64_t m) {
 // partitions whose build side fits one table. Under a budget and with
 // per-stage timing the pipeline runs as ever.
 bool may_run_direct(const vj_ctx *c, const Plan &pl) {
-    if (!pl.fan || pl.joins.size() != 1 || pl.any_part || c->budget || c->profiling || !c->direct || !c->na_stage) return false;
+    if (!pl.fan || pl.joins.size() != 1 || pl.any_part || c->budget || c->profiling || c->by_events || !c->direct || !c->na_stage) return false;
     const JobDesc &r = pl.jobs[pl.joins[0].job_r], &s = pl.jobs[pl.joins[0].job_s];
     return !r.b1 && !s.b1 && r.n > 0 && s.n > 0 && r.n <= pl.joins[0].cap_r;
 }
@@ -1239,9 +1248,7 @@ Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std:
         a.out_r = js.out_r;
         a.out_s = js.out_s;
         a.cap = js.cap;
-        VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
         VJ_LAUNCH(launch_flat(a, sh, s));
-        VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
         VJ_HIP_TRY(hipStreamSynchronize(s));
         if (a.down[0] & kFlatGiveUp) {
             c->flat_skip[tune_key(a.r.n, kb, sh.hp)] = 64;
@@ -1262,7 +1269,7 @@ Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std:
     sm.retries = retries;
     sm.partitions = 1;
     sm.tasks = 1;
-    sm.ms_total = elapsed(c->ev[EV_START], c->ev[EV_PROBE]);
+    sm.ms_total = clock_ms(c, a.down[1], a.down[2]);
     sm.scratch_bytes = held_bytes(c);
     sm.tile_rows = pass_tile(kb, 0);
     sm.probe_threads = kFlatThreads;
@@ -1380,9 +1387,7 @@ Err run_direct(vj_ctx *c, Plan &pl, JoinSpec &js, hipStream_t s, std::vector<uin
         d.out_r = js.out_r;
         d.out_s = js.out_s;
         d.cap = js.cap;
-        VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
         VJ_LAUNCH(launch_direct(d, pl.shape, blocks, s));
-        VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
         VJ_HIP_TRY(hipStreamSynchronize(s));
         if (!grow || down[0] <= js.cap) break;
         VJ_TRY(regrow(c, js, down[0]));
@@ -1390,7 +1395,7 @@ Err run_direct(vj_ctx *c, Plan &pl, JoinSpec &js, hipStream_t s, std::vector<uin
     }
     counts.assign(1, down[0]);
     if (retries_out) *retries_out = retries;
-    fill_summary(c, pl, js, counts[0], (uint64_t)blocks, retries, false, held_bytes(c));
+    fill_summary(c, pl, js, counts[0], (uint64_t)blocks, retries, false, held_bytes(c), down[1], down[2]);
     return Err::ok();
 }
 
@@ -1447,9 +1452,10 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
     }
     if (replay) {
         stage_descriptors(static_cast<char *>(c->pinned), pl);  // the graph's upload node reads them at launch
-        VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
+        const bool events = !timed_by_clock(c, pl);
+        if (events) VJ_HIP_TRY(hipEventRecord(c->ev[EV_START], s));
         VJ_HIP_TRY(hipGraphLaunch(c->graph, s));
-        VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
+        if (events) VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
         c->graph_replays++;
     } else {
         VJ_TRY(upload(ctx_arenas(c), pl, s));
@@ -1493,15 +1499,16 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
                                       pl.joins.size() * sizeof(JoinDesc), hipMemcpyHostToDevice, s));
             VJ_LAUNCH(launch_reset_probe(a, s));
             VJ_LAUNCH(launch_probe(a, pl.shape, probe_grid(c, pl), s));
-            VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
+            if (!timed_by_clock(c, pl)) VJ_HIP_TRY(hipEventRecord(c->ev[EV_PROBE], s));
             VJ_HIP_TRY(hipStreamSynchronize(s));
             counts.assign(hc, hc + pl.joins.size());
         }
     }
     if (retries_out) *retries_out = retries;
-    if (specs.size() == 1)
-        fill_summary(c, pl, specs[0], counts[0], reinterpret_cast<const Ctl *>(h + pl.off_ctl)->task_total, retries,
-                     replay, held_bytes(c));
+    if (specs.size() == 1) {
+        const Ctl *ctl = reinterpret_cast<const Ctl *>(h + pl.off_ctl);
+        fill_summary(c, pl, specs[0], counts[0], ctl->task_total, retries, replay, held_bytes(c), ctl->t0, ctl->t1);
+    }
     return Err::ok();
 }
 
@@ -1592,6 +1599,10 @@ vj_status vj_ctx_create(int device, vj_ctx **out) {
     vj_ctx *c = new vj_ctx();
     c->device = device;
     c->cus = device_cu_count(device);
+    if (hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, device) != hipSuccess) {
+        (void)hipGetLastError();
+        c->clock_khz = 0;
+    }
     for (int i = 0; i < EV_COUNT; i++) {
         if (hipEventCreate(&c->ev[i]) != hipSuccess) {
             for (int k = 0; k < i; k++) (void)hipEventDestroy(c->ev[k]);
@@ -1742,8 +1753,8 @@ vj_status vj_join_into_noalloc(vj_ctx *c, const vj_table *build, const vj_table 
     }
     if (e.failed()) return fail(c, e);
     const uint64_t m = *reinterpret_cast<const unsigned long long *>(ar.pinned + pl.off_count);
-    fill_summary(c, pl, specs[0], m, reinterpret_cast<const Ctl *>(ar.pinned + pl.off_ctl)->task_total, 0, false,
-                 az.sum());
+    const Ctl *ctl = reinterpret_cast<const Ctl *>(ar.pinned + pl.off_ctl);
+    fill_summary(c, pl, specs[0], m, ctl->task_total, 0, false, az.sum(), ctl->t0, ctl->t1);
     *count = m;
     if (m > capacity)
         return fail(c, Err::make(VJ_ERR_CAPACITY, "output holds " + std::to_string(capacity) + " pairs, join has " +
@@ -2143,7 +2154,9 @@ vj_status vj_tune(vj_ctx *c, const vj_table *build, const vj_table *probe, const
         const vj_join_opts o2 = plan_opts(x);
         std::vector<double> ts;
         for (int r = 0; r <= reps; r++) {  // the first run warms the arenas
+            c->by_events = true;
             Err er = run_joins(c, specs, &o2, s, counts, false, 0, nullptr);
+            c->by_events = false;
             if (er.failed()) return er;
             if (r) ts.push_back(c->summary.ms_total);
         }

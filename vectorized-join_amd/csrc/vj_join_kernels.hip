@@ -366,6 +366,7 @@ __global__ __launch_bounds__(1024) void k_fan_begin(PipeArgs a) {
         a.ctl->task_ticket = 0;
         a.ctl->overflow = 0;
         a.ctl->done = 0;
+        a.ctl->t0 = wall_clock64();
     }
     for (uint32_t i = i0; i < a.up_words; i += step) a.up_dst[i] = a.up_src[i];
     const gptr<uint32_t> c = to_global(a.counts);
@@ -515,6 +516,7 @@ __global__ __launch_bounds__(256) void k_stage_copy(unsigned long long *dst, con
 __global__ __launch_bounds__(256) void k_flat_begin(FlatArgs a) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const gptr<u32x4> t = (gptr<u32x4>)a.slots;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.count[1] = wall_clock64();
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.zero_words; i += gridDim.x * 256) t[i] = u32x4{0, 0, 0, 0};
 }
 

@@ -202,11 +202,14 @@ struct ColScanDesc {
 // build+probe kernel reads them. overflow: a region of the region layout
 // received more rows than it holds (set by k_tasks).
 // done: build+probe blocks that have ended; the last one sets it back to 0.
+// t0, t1: the device clock at the start of the first kernel (one-pass form) and
+// at the end of the last block (written to the host's copy only).
 struct Ctl {
     unsigned long long task_ticket;
     unsigned long long task_total;
     unsigned long long overflow;
     unsigned long long done;
+    unsigned long long t0, t1;
 };
 
 
@@ -238,14 +241,15 @@ struct PipeArgs {
     unsigned long long *up_dst;
     const unsigned long long *up_src;
     uint32_t up_words;
-    // out_count and what follows it (to the end of ctl) goes to the host's buffer when build+probe ends
+    // out_count and what follows it (to ctl's t0; t1 is taken then) goes to the host's buffer when build+probe ends
     uint32_t down_words;
     unsigned long long *down;
     HashCfg hash;
 };
 
 // One join without partitions (k_direct). count and done are zero before the
-// launch and after it; the match count is written to `down` (host memory).
+// launch and after it; the match count and the device clock at the start
+// (count[1]) and the end are written to `down` (host memory).
 struct DirectArgs {
     TView r, s;
     uint32_t *out_r, *out_s;
