@@ -1241,7 +1241,7 @@ Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std:
     a.nxt = reinterpret_cast<uint32_t *>(m + table + kAlign);
     a.zero_words = (uint32_t)((table + 16) / 16);
     a.count = static_cast<unsigned long long *>(c->direct);
-    a.done = a.count + 32;
+    a.clock = a.count + 1;
     a.down = static_cast<unsigned long long *>(c->na_stage);
     int retries = 0;
     while (true) {
@@ -1272,7 +1272,7 @@ Err run_flat(vj_ctx *c, JoinSpec &js, const vj_join_opts *o, hipStream_t s, std:
     sm.ms_total = clock_ms(c, a.down[1], a.down[2]);
     sm.scratch_bytes = held_bytes(c);
     sm.tile_rows = pass_tile(kb, 0);
-    sm.probe_threads = kFlatThreads;
+    sm.probe_threads = a.s.n <= 1u << 18 ? 512 : 1024;
     sm.table_rows = (int32_t)a.r.n;
     sm.layout = VJ_LAYOUT_EXACT;
     sm.bytes_build_probe = a.r.n * (kb + (a.r.rowids ? 4u : 0u)) + a.s.n * (kb + (a.s.rowids ? 4u : 0u)) + counts[0] * 8;
@@ -1327,7 +1327,7 @@ Err run_flat_batch(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_
     const size_t dups = align_up(n * 4);
     VJ_TRY(ensure(c->tuples, tables + dups + links, true));
     const size_t o_b0 = align_up(n * sizeof(FlatArgs)), o_p0 = align_up(o_b0 + (n + 1) * 4), up = align_up(o_p0 + (n + 1) * 4);
-    const size_t o_counts = up, o_done = align_up(o_counts + n * 8), meta = o_done + kAlign;
+    const size_t o_counts = up, meta = align_up(o_counts + n * 8);
     VJ_TRY(ensure(c->meta, meta, true));
     VJ_TRY(ensure_pinned(c, meta));
     char *m = static_cast<char *>(c->tuples.p), *d = static_cast<char *>(c->meta.p), *p = static_cast<char *>(c->pinned);
@@ -1345,20 +1345,21 @@ Err run_flat_batch(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_
     b.zero = reinterpret_cast<uint32_t *>(m);
     b.zero_words = (tables + dups) / 16;
     b.counts = reinterpret_cast<unsigned long long *>(d + o_counts);
-    b.done = reinterpret_cast<unsigned long long *>(d + o_done);
-    b.down = reinterpret_cast<unsigned long long *>(p + o_counts);
+    unsigned long long *down = reinterpret_cast<unsigned long long *>(p + o_counts);
     for (size_t i = 0; i < n; i++) {
         args[i].slots = reinterpret_cast<uint32_t *>(m + at[i]);
         args[i].dup = reinterpret_cast<uint32_t *>(m + tables) + i;
         args[i].nxt = reinterpret_cast<uint32_t *>(m + tables + dups + links_at[i]);
         args[i].count = b.counts + i;
+        args[i].down = down + i;
+        down[i] = 0;  // a join with an empty side has no block to write it
     }
     memcpy(p, args.data(), n * sizeof(FlatArgs));
     memcpy(p + o_b0, build0.data(), (n + 1) * 4);
     memcpy(p + o_p0, probe0.data(), (n + 1) * 4);
     VJ_LAUNCH(launch_flat_batch(b, sh, s));
     VJ_HIP_TRY(hipStreamSynchronize(s));
-    counts.assign(b.down, b.down + n);
+    counts.assign(down, down + n);
     for (uint64_t x : counts) {
         if (x & kFlatGiveUp) {
             c->flat_skip[tune_key(largest_build(specs), kb, sh.hp)] = 64;

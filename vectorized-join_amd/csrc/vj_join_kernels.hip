@@ -516,7 +516,7 @@ __global__ __launch_bounds__(256) void k_stage_copy(unsigned long long *dst, con
 __global__ __launch_bounds__(256) void k_flat_begin(FlatArgs a) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const gptr<u32x4> t = (gptr<u32x4>)a.slots;
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.count[1] = wall_clock64();
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.clock = wall_clock64();
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.zero_words; i += gridDim.x * 256) t[i] = u32x4{0, 0, 0, 0};
 }
 
@@ -526,7 +526,6 @@ __global__ __launch_bounds__(256) void k_flat_begin_batch(FlatBatch b) {
     const uint32_t i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
     for (uint32_t i = i0; i < b.up_words; i += step) b.up_dst[i] = b.up_src[i];
     for (uint32_t j = i0; j < b.n_joins; j += step) b.counts[j] = 0;
-    if (i0 == 0) *b.done = 0;
     const gptr<u32x4> t = (gptr<u32x4>)b.zero;
     for (uint64_t i = i0; i < b.zero_words; i += step) t[i] = u32x4{0, 0, 0, 0};
 }

@@ -1293,8 +1293,12 @@ template <int HP, int KW, int NC> __global__ __launch_bounds__(kFlatThreads) voi
     flat_build_block<HP, KW, NC>(a, blockIdx.x);
 }
 
-template <int HP, int KW, int NC, int U> __device__ __forceinline__ void flat_probe_block(const FlatArgs &a, uint32_t block) {
-    constexpr int WAVES = kFlatThreads / 64;
+// `blocks`: of the join. One atomic per block reserves its output rows and
+// counts it (kFlatBlock): the last block to reserve knows the join's count and
+// hands it to the host, with the device clock.
+template <int HP, int KW, int NC, int TH, int U>
+__device__ __forceinline__ void flat_probe_block(const FlatArgs &a, uint32_t block, uint32_t blocks) {
+    constexpr int WAVES = TH / 64;
     constexpr bool K4 = KW * NC == 4, WIDE = KW * NC > 8;
     __shared__ uint32_t wave_count[WAVES];
     __shared__ unsigned long long out_base;
@@ -1308,7 +1312,7 @@ template <int HP, int KW, int NC, int U> __device__ __forceinline__ void flat_pr
     const uint32_t n = (uint32_t)a.s.n, mask = a.mask, hshift = a.hshift;
     const bool dup = *a.dup != 0;
     // a wave's rows are consecutive, and so are its matches
-    const uint32_t row0 = block * (kFlatThreads * U) + w * 64 * U + lane;
+    const uint32_t row0 = block * (TH * U) + w * 64 * U + lane;
     Key<KW, NC> k[U];
 #pragma unroll
     for (int u = 0; u < U; u++) k[u] = load_key<KW, NC>(sk, row0 + u * 64 < n ? row0 + u * 64 : 0u);
@@ -1368,10 +1372,18 @@ template <int HP, int KW, int NC, int U> __device__ __forceinline__ void flat_pr
         uint32_t sum = 0;
         for (int x = 0; x < WAVES; x++) sum += wave_count[x];
         // A key with too many rows to follow one by one: the host runs the join in the pipeline (with the top
-        // bit of the count set no reservation is below any capacity, so nothing more is written). Both atomics
-        // are waited for here: this thread counts the block as ended after them.
-        if (long_chain) out_base = atomicOr(a.count, kFlatGiveUp) | kFlatGiveUp;
-        else out_base = sum ? atomicAdd(a.count, (unsigned long long)sum) : 0;
+        // bit of the count set nothing more is written).
+        const unsigned long long gave_up = long_chain ? atomicOr(a.count, kFlatGiveUp) | kFlatGiveUp : 0;
+        const unsigned long long got = atomicAdd(a.count, kFlatBlock | sum) | (gave_up & kFlatGiveUp);
+        out_base = got & kFlatGiveUp ? kFlatGiveUp : got & (kFlatBlock - 1);
+        if ((uint32_t)((got & ~kFlatGiveUp) / kFlatBlock) + 1 == blocks) {
+            a.down[0] = (got & kFlatGiveUp) | ((got & (kFlatBlock - 1)) + sum);
+            if (a.clock) {  // a single join; its counter is zero again for the next one
+                a.down[1] = *a.clock;
+                a.down[2] = wall_clock64();
+                *a.count = 0;
+            }
+        }
     }
     const gptr<const uint32_t> rid = uniform_global(a.r.rowids), sid = uniform_global(a.s.rowids);
     uint32_t r[U], s[U];
@@ -1417,13 +1429,8 @@ template <int HP, int KW, int NC, int U> __device__ __forceinline__ void flat_pr
     }
 }
 
-template <int HP, int KW, int NC, int U> __global__ __launch_bounds__(kFlatThreads) void k_flat_probe(FlatArgs a) {
-    __shared__ uint32_t last;
-    flat_probe_block<HP, KW, NC, U>(a, blockIdx.x);
-    if (finish_block(last, a.done, a.count, a.down, 2)) {
-        __syncthreads();
-        if (threadIdx.x == 0) *a.count = 0;  // for the next join
-    }
+template <int HP, int KW, int NC, int TH, int U> __global__ __launch_bounds__(TH) void k_flat_probe(FlatArgs a) {
+    flat_probe_block<HP, KW, NC, TH, U>(a, blockIdx.x, gridDim.x);
 }
 
 // A batch's blocks stand join after join in one line, of which each XCD takes
@@ -1444,11 +1451,9 @@ template <int HP, int KW, int NC> __global__ __launch_bounds__(kFlatThreads) voi
 }
 
 template <int HP, int KW, int NC> __global__ __launch_bounds__(kFlatThreads) void k_flat_probe_batch(FlatBatch b) {
-    __shared__ uint32_t last;
     uint32_t j, block;
     if (flat_batch_at(b.probe0, b.n_joins, b.probe_blocks, j, block))
-        flat_probe_block<HP, KW, NC, flat_batch_rows(KW * NC)>(b.joins[j], block);
-    (void)finish_block(last, b.done, b.counts, b.down, b.n_joins);
+        flat_probe_block<HP, KW, NC, kFlatThreads, flat_batch_rows(KW * NC)>(b.joins[j], block, b.probe0[j + 1] - b.probe0[j]);
 }
 
 // Dispatch over the key shape (key width, key columns).
@@ -1560,17 +1565,18 @@ template <int HP> hipError_t StageLaunch<HP>::direct(const DirectArgs &d, const 
 
 template <int HP> hipError_t StageLaunch<HP>::flat(const FlatArgs &a, const LaunchShape &sh, hipStream_t s) {
     return dispatch_keys(sh, [&]<int KW, int NC>() {
-        constexpr int U = KW * NC <= 8 ? 8 : 4;
         const uint32_t n = (uint32_t)a.s.n;
         hipLaunchKernelGGL((k_flat_build<HP, KW, NC>), dim3(((uint32_t)a.r.n + kFlatThreads - 1) / kFlatThreads), dim3(kFlatThreads), 0, s, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        // few probe rows: fewer per thread, so that more CUs take part
-        if (n <= 1u << 20)
-            hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, 2>), dim3((n - 1) / (kFlatThreads * 2) + 1), dim3(kFlatThreads), 0, s, a);
-        else
-            hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, U>), dim3((n - 1) / (kFlatThreads * U) + 1), dim3(kFlatThreads), 0, s, a);
-        return hipGetLastError();
+        auto probe = [&]<int TH, int U>() {
+            hipLaunchKernelGGL((k_flat_probe<HP, KW, NC, TH, U>), dim3((n - 1) / (TH * U) + 1), dim3(TH), 0, s, a);
+            return hipGetLastError();
+        };
+        // the largest blocks that leave no CU without one
+        if (n <= 1u << 18) return probe.template operator()<512, 2>();
+        if (n <= 1u << 19) return probe.template operator()<1024, 2>();
+        return probe.template operator()<1024, 4>();
     });
 }
 

@@ -263,8 +263,19 @@ struct DirectArgs {
 // The flat form (k_flat_build, k_flat_probe): slots of the table in 16-byte
 // groups, zero before the build; links of equal keys, one per build row.
 constexpr int kFlatThreads = 512;
+// Probe blocks of a single join are large, since every block takes a turn at the
+// one counter (join_into, us: 2^16 x 2^20 4-byte keys 51 with two atomics per
+// block of 512 x 2 rows, 47 with one, 40 with one per 1024 x 4; 2^18 x 2^24,
+// 512 x 8: 167, 1024 x 4: 161; 2^16 x 2^22 8-byte keys 94 / 90; 2^18 probe rows
+// 4 x u32, 512 x 2: 81, 1024 x 2: 84). A batch's are of kFlatThreads and these rows
+// per thread: its counters are as many as its joins (64 joins of up to 2048 int64
+// rows, 512 x 8: 90, 1024 x 4: 103).
+__host__ __device__ constexpr int flat_batch_rows(int key_bytes) { return key_bytes <= 8 ? 8 : 4; }
 constexpr uint32_t kFlatChain = 64;                     // rows of one key followed link by link
 constexpr unsigned long long kFlatGiveUp = 1ull << 63;  // in the count: a chain was longer
+// The counter of a join: matches (below 2^32 rows x 65) and, above them, the
+// blocks that have reserved their output (at most 2^22 of 1024 rows or more).
+constexpr unsigned long long kFlatBlock = 1ull << 40;
 constexpr uint64_t kFlatTableBytes = 4ull << 20;  // an XCD's L2
 // All tables of a batch, beyond which the pipeline is the faster one (us a call,
 // flat and pipeline, build sides log-uniform from 2^10, probe sides 4-16 times
@@ -283,8 +294,6 @@ __host__ __device__ constexpr int flat_slot_bytes(int key_bytes) { return key_by
 __host__ __device__ constexpr uint64_t flat_max_rows(int key_bytes) {
     return kFlatTableBytes / flat_slot_bytes(key_bytes) / (key_bytes <= 4 ? 2 : 4);
 }
-// Probe rows per thread of a batch's joins.
-__host__ __device__ constexpr int flat_batch_rows(int key_bytes) { return key_bytes <= 8 ? 8 : 4; }
 struct FlatArgs {
     TView r, s;
     uint32_t *slots;
@@ -296,7 +305,9 @@ struct FlatArgs {
     uint64_t cap;
     uint32_t one_based;
     uint32_t zero_words;  // 16-byte words from `slots` on to clear before the build (the table, then dup)
-    unsigned long long *count, *done, *down;  // as DirectArgs
+    // the counter, zero before the launch (and after it where clock is set); host memory for the match count
+    // (then the device clock at the start and the end); a single join's start on that clock
+    unsigned long long *count, *down, *clock;
     HashCfg hash;
 };
 
@@ -311,7 +322,7 @@ struct FlatBatch {
     const unsigned long long *up_src;
     uint32_t *zero;                   // the tables and their dup words
     uint64_t zero_words;              // in 16-byte words
-    unsigned long long *counts, *done, *down;
+    unsigned long long *counts;
 };
 
 // Kernel launchers (vj_join_kernels.hip); all asynchronous on `s`.
