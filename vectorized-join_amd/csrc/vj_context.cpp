@@ -1410,8 +1410,23 @@ enum GraphMode { GRAPH_OFF, GRAPH_ON, GRAPH_AUTO };
 Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hipStream_t s,
               std::vector<uint64_t> &counts, bool grow, uint64_t extra_bytes, int *retries_out,
               GraphMode gmode = GRAPH_OFF) {
+    // Row-major keys: columns before anything else reads them, except where the
+    // one-pass form's histogram makes them
+    const bool from_rows = specs.size() == 1 && (specs[0].r_rows || specs[0].s_rows);
+    auto to_cols = [&]() -> Err {
+        if (!from_rows) return Err::ok();
+        JoinSpec &js = specs[0];
+        for (int k = 0; k < 2; k++) {
+            const vj_table *t = k ? js.s : js.r;
+            const uint64_t *rows = k ? js.s_rows : js.r_rows;
+            if (rows) VJ_TRY(launch_rows_to_cols(rows, t->n_rows, t->n_cols, static_cast<uint64_t *>(const_cast<void *>(t->cols[0])), s, c->cus));
+        }
+        js.r_rows = js.s_rows = nullptr;
+        return Err::ok();
+    };
     if (may_run_flat(c, specs, o)) {
         bool ran = false;
+        VJ_TRY(to_cols());
         VJ_TRY(run_flat(c, specs[0], o, s, counts, grow, retries_out, &ran));
         if (ran) return Err::ok();
     }
@@ -1423,6 +1438,15 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
     }
     Plan pl;
     VJ_TRY(plan_joins(pl, specs, o, c, true, c->budget != 0));
+    if (from_rows && (specs[0].r_rows || specs[0].s_rows)) {
+        JobDesc &jr = pl.jobs[pl.joins[0].job_r], &jsd = pl.jobs[pl.joins[0].job_s];
+        if (pl.fan && jr.nrow && jsd.nrow) {  // both sides have a histogram
+            jr.mid_cols[0] = const_cast<uint64_t *>(specs[0].r_rows);
+            jsd.mid_cols[0] = const_cast<uint64_t *>(specs[0].s_rows);
+        } else {
+            VJ_TRY(to_cols());
+        }
+    }
     if (may_run_direct(c, pl)) return run_direct(c, pl, specs[0], s, counts, grow, retries_out);
     VJ_TRY(admit(c, pl, extra_bytes + pl.keep_bytes));
     VJ_TRY(allocate(c, pl));
@@ -1517,11 +1541,13 @@ Err run_joins(vj_ctx *c, std::vector<JoinSpec> &specs, const vj_join_opts *o, hi
 // rows), regrown when the join has more pairs. `held_extra` is device memory
 // the caller already holds for this join (counted against the budget).
 Err join_callee_alloc(vj_ctx *c, const vj_table *build, const vj_table *probe, const vj_join_opts *opts, hipStream_t s,
-                      uint64_t held_extra, vj_pairs *out) {
+                      uint64_t held_extra, vj_pairs *out, const uint64_t *r_rows = nullptr, const uint64_t *s_rows = nullptr) {
     const uint64_t cap = opts->out_capacity_hint ? opts->out_capacity_hint : std::max<uint64_t>(probe->n_rows, 1);
     if (c->budget && cap * 8 + held_extra > c->budget)  // the output alone breaks the budget: nothing is allocated
         return Err::make(VJ_ERR_BUDGET, "an output of " + std::to_string(cap) + " pairs exceeds the HBM budget");
     std::vector<JoinSpec> specs{{build, probe, nullptr, nullptr, cap}};
+    specs[0].r_rows = r_rows;
+    specs[0].s_rows = s_rows;
     if (alloc_ids(c, &specs[0].out_r, cap) != hipSuccess || alloc_ids(c, &specs[0].out_s, cap) != hipSuccess) {
         cache_free(specs[0].out_r, true);
         return Err::make(VJ_ERR_OUT_OF_MEMORY, "output allocation failed");
@@ -1801,7 +1827,7 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
     hipStream_t st = (hipStream_t)stream;
     const int nc = r->n_cols;
     // Key columns for the pipeline: one column of a row-major table is already
-    // contiguous; wider rows are transposed into temporary columns.
+    // contiguous; wider rows are transposed into temporary columns, by the run.
     uint64_t *tmp = nullptr;
     const uint64_t tmp_words = nc > 1 ? (r->n_rows + s->n_rows) * (uint64_t)nc : 0;
     if (tmp_words) {
@@ -1810,8 +1836,6 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
         if (cache_malloc(reinterpret_cast<void **>(&tmp), tmp_words * 8, c->budget == 0) != hipSuccess) {
             return fail(c, Err::make(VJ_ERR_OUT_OF_MEMORY, "hipMalloc of the transposed key columns failed"));
         }
-        e = launch_rows_to_cols(r->column_values, r->n_rows, nc, tmp, st, c->cus);
-        if (!e.failed()) e = launch_rows_to_cols(s->column_values, s->n_rows, nc, tmp + r->n_rows * nc, st, c->cus);
     }
     vj_table rt{}, stt{};
     for (int k = 0; k < 2; k++) {
@@ -1824,7 +1848,9 @@ vj_status vj_join_rows(vj_ctx *c, const vj_rows *r, const vj_rows *s, const vj_j
         for (int cc = 0; cc < nc; cc++) t.cols[cc] = nc > 1 ? base + (uint64_t)cc * src->n_rows : base;
     }
     vj_pairs pairs{};
-    if (!e.failed()) e = join_callee_alloc(c, &rt, &stt, opts, st, tmp_words * 8, &pairs);
+    if (!e.failed())
+        e = join_callee_alloc(c, &rt, &stt, opts, st, tmp_words * 8, &pairs, tmp ? r->column_values : nullptr,
+                              tmp ? s->column_values : nullptr);
     const uint64_t m = pairs.count;
     if (!e.failed() && m) {  // rs: (r pk, s pk) per pair, row-major, and primary keys 1..M
         if (c->budget && held_bytes(c) + tmp_words * 8 + m * 8 + m * 24 > c->budget) {

@@ -31,6 +31,8 @@ struct JoinSpec {
     uint64_t cap;
     const vj_built *res = nullptr;  // probe this resident build side (r unused)
     vj_built *keep = nullptr;       // keep r's partitioned rows here (allocated by the run)
+    // row-major 64-bit keys that r's / s's columns (temporary ones) are yet to be filled from
+    const uint64_t *r_rows = nullptr, *s_rows = nullptr;
 };
 
 // Device bytes a pipeline over `specs` needs: context scratch (with the

@@ -390,9 +390,13 @@ __device__ __forceinline__ uint32_t fan_part(uint32_t h, uint32_t b1, uint32_t b
 
 // Rows per (group, partition). Each block sweeps every nper-th tile of one
 // group with one LDS atomic per row, then adds its counters to the job's.
-// HBM-bound: the keys once.
+// HBM-bound: the keys once. Row-major keys (vj_join_rows) become columns on the
+// way: as a kernel of its own in front this read them once more and took two
+// launches (us a call with its consumer, before and now: 2^20 x 2^22 rows of 2 columns
+// 343 / 325, of 3 390 / 362, 70000 x 300000 of 2 155 / 133).
 template <int HP, int KW, int NC>
 __global__ __launch_bounds__(kFanThreads, 8) void k_fan_hist(PipeArgs a) {
+    using KT = typename KeyT<KW>::T;
     constexpr int KB = KW * NC;
     constexpr int U = KB <= 16 ? 4 : 2;  // rows per thread in flight
     extern __shared__ uint32_t lds[];    // [2^(b1+b2)]
@@ -405,6 +409,7 @@ __global__ __launch_bounds__(kFanThreads, 8) void k_fan_hist(PipeArgs a) {
     __syncthreads();
     const GKeys<KW, NC> in = uniform_keys<KW, NC>(job.in);
     const HashCfg hc = a.hash;
+    [[maybe_unused]] const gptr<const uint64_t> rows = uniform_global(static_cast<const uint64_t *>(job.mid_cols[0]));
     const uint32_t T = a.pass_tile, tiles = job.p1_tiles;
     // the group's tiles: those whose index over the whole pipeline is g modulo the group count
     for (uint32_t t = ((g - a.p1_tile0[j]) & (G - 1)) + G * (local / G); t < tiles; t += G * nper) {
@@ -414,7 +419,26 @@ __global__ __launch_bounds__(kFanThreads, 8) void k_fan_hist(PipeArgs a) {
 #pragma unroll
             for (int u = 0; u < U; u++) {  // all loads in flight at once (past the end: the first row again)
                 const uint32_t i = i0 + u * kFanThreads;
-                key[u] = load_key<KW, NC>(in, i < hi ? i : i0);
+                const uint64_t r = i < hi ? i : i0;
+                if constexpr (KW == 8 && NC > 1) {
+                    if (rows) {  // block-uniform
+#pragma unroll
+                        for (int c = 0; c < NC; c++) key[u].c[c] = rows[r * NC + c];
+                        continue;
+                    }
+                }
+                key[u] = load_key<KW, NC>(in, r);
+            }
+            if constexpr (KW == 8 && NC > 1) {
+                if (rows) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const uint32_t i = i0 + u * kFanThreads;
+#pragma unroll
+                        for (int c = 0; c < NC; c++)
+                            if (i < hi) ((gptr<KT>)in.c[c])[i] = key[u].c[c];
+                    }
+                }
             }
 #pragma unroll
             for (int u = 0; u < U; u++)

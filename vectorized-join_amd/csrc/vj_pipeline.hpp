@@ -137,7 +137,9 @@ static_assert(probe_table_bytes(8, 1) <= kTableBytes && probe_table_bytes(8, 2) 
 
 struct JobDesc {
     TView in;                 // the caller's table
-    void *mid_cols[4];        // pass-1 output (2-pass jobs)
+    // pass-1 output (2-pass jobs); one-pass form: [0] is null, or row-major 64-bit
+    // keys that k_fan_hist reads in place of in's columns, which it fills
+    void *mid_cols[4];
     uint32_t *mid_ids;
     void *fin_cols[4];        // last-pass output (partitioned jobs)
     uint32_t *fin_ids;

@@ -9,7 +9,8 @@
 // matching pair, with primary keys 1..M.
 //
 //   k_rows_to_cols  row-major n x C u64 keys -> C SoA columns (C = 2..4), so the
-//                   pipeline reads each key column contiguously
+//                   pipeline reads each key column contiguously; where the
+//                   join takes the one-pass form its histogram does this
 //   k_materialize   (build row, probe row) index pairs -> the reference's rs
 //                   rows (one 16-byte store per pair) and primary keys 1..M
 // Both are HBM-bound: the transpose moves 2 x 8C bytes per row; the
