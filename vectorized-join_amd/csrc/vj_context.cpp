@@ -1175,24 +1175,25 @@ bool flat_class_ok(vj_ctx *c, uint64_t key) {
 }
 
 // Whether a join runs in the flat form: a single join whose build side is
-// past an LDS table and whose table an XCD's L2 holds.
+// past an LDS table and whose table an XCD's L2 holds, or nearly so (flat_max_rows).
 bool may_run_flat(vj_ctx *c, const std::vector<JoinSpec> &specs, const vj_join_opts *o) {
     if (!flat_allowed(c, o) || specs.size() != 1 || specs[0].res || specs[0].keep) return false;
     const vj_table *r = specs[0].r, *s = specs[0].s;
     const int kb = s->key_width * s->n_cols;
-    if (r->n_rows <= (uint64_t)build_cap(kb) * 3 / 4 || r->n_rows > flat_max_rows(kb) || s->n_rows == 0) return false;
+    if (r->n_rows <= (uint64_t)build_cap(kb) * 3 / 4 || s->n_rows == 0) return false;
+    const bool past_l2 = kb > 4 && r->n_rows <= 2 * flat_max_rows(kb) && s->n_rows >= r->n_rows && s->n_rows <= kFlatMaxProbe;
+    if (r->n_rows > flat_max_rows(kb) && !past_l2) return false;
     HashCfg h;
     if (make_hash_cfg(&o->hash, s, &h).failed()) return false;
     return flat_class_ok(c, tune_key(r->n_rows, kb, hash_path(h)));
 }
 
-// Slots of the table of n build rows: a quarter full where that still fits, else
-// up to half; in a batch single slots are a quarter full, and pairs half, as more
-// tables share an L2. At least two pairs: the kernels shift a 32-bit product by 32
+// Slots of the table of n build rows: single ones a quarter full, pairs too where
+// that still fits an L2, else (and in a batch, whose tables share it) up to half. At least two pairs: the kernels shift a 32-bit product by 32
 // less their log2.
 uint64_t flat_slots(uint64_t n, int kb, bool batch) {
     const uint64_t slots = std::max<uint64_t>(4, 1ull << ceil_log2(2 * n));
-    return batch && kb <= 4 ? slots : slots * 2 * flat_slot_bytes(kb) <= kFlatTableBytes ? slots * 2 : slots;
+    return kb > 4 || (!batch && slots * 2 * flat_slot_bytes(kb) <= kFlatTableBytes) ? slots * 2 : slots;
 }
 
 // The kernels' arguments of one join but for its memory.

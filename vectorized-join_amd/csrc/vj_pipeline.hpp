@@ -290,12 +290,17 @@ constexpr uint64_t kFlatTableBytes = 4ull << 20;  // an XCD's L2
 __host__ __device__ constexpr uint64_t flat_batch_bytes(int key_bytes) { return (key_bytes > 4 && key_bytes <= 8 ? 16ull : 32ull) << 20; }
 __host__ __device__ constexpr int flat_slot_bytes(int key_bytes) { return key_bytes <= 4 ? 8 : 16; }
 // Build rows of the largest table: half full in pairs of 8-byte slots, a
-// quarter in single 16-byte ones, whose chains grow sooner (device us, flat and
-// pipeline: 2^18 x 2^24 4-byte keys 147 / 166; 2^16 x 2^20 8-byte keys 46 / 61,
-// 4 x u32 50 / 81; 2^17 x 2^20 8-byte keys, half full, 96 / 62).
+// quarter in single 16-byte ones, whose chains grow sooner (join_into, us, flat and
+// pipeline: 4-byte keys 2^18 x 2^24 162 / 180, 2^19 x 2^22 108 / 92; 8-byte keys
+// 2^16 x 2^20 52 / 76, 2^16 x 2^22 85 / 100; 4 x u32 2^16 x 2^20 65 / 114). Twice
+// as many rows of over 4 bytes, a table past an L2, where the probe side is of the
+// build side's size or more and not past kFlatMaxProbe rows: 8-byte keys 2^17 x 2^20
+// 65 / 74, 2^17 x 2^22 110 / 98, 2^18 x 2^20 84 / 75; 4 x u32 2^17 x 2^20 74 / 89,
+// 2^17 x 2^22 162 / 136; 4 x u64 2^17 x 2^21 132 / 141.
 __host__ __device__ constexpr uint64_t flat_max_rows(int key_bytes) {
     return kFlatTableBytes / flat_slot_bytes(key_bytes) / (key_bytes <= 4 ? 2 : 4);
 }
+constexpr uint64_t kFlatMaxProbe = 1ull << 21;
 struct FlatArgs {
     TView r, s;
     uint32_t *slots;
